@@ -4,10 +4,9 @@
 // loop of ForwardBatch (:473-488) layer by layer.
 //
 // Per layer, on one stream (x [T, dim] is the residual stream, in place;
-// for 1 and for 2..32 tokens with quantized weights q/k/v are one launch,
-// gate/up carry the SwiGLU and the down projection adds into x; for many
-// tokens over Q8_0 / Q4_0 blocks gate/up carry the SwiGLU, wo and down add
-// into x and k, v may share one launch; with separate q/k/v launches at
+// for 1 and for 2..32 tokens with quantized weights, and for more than 32
+// with any, q/k/v are one launch, gate/up carry the SwiGLU and wo or the
+// down projection add into x; with q/k/v not rotated in their launch, at
 // consecutive positions k and v are written to their cache rows and
 // rotated there, with no copy; see below):
 //   h = RmsNorm(x, attention_norm)                    mlk_rmsnorm_f32
@@ -61,6 +60,11 @@ bool FusedRows(int64_t T) { return T >= 8 && T <= 32; }
 // bf16 kernel, fused as FusedRows; one token keeps the block-layout GEMVs).
 bool PlanarRows(int64_t T) { return T >= 2 && T <= 32; }
 
+struct TileGroup {
+    int64_t in, rows[3];
+    int n;
+};
+
 Plan MakePlan(const mlk_layer_config& c, int64_t T, int64_t max_ctx, bool contiguous) {
     const int64_t D = c.dim, F = c.hidden_dim;
     const int64_t QD = static_cast<int64_t>(c.n_heads) * c.head_dim;
@@ -83,6 +87,11 @@ Plan MakePlan(const mlk_layer_config& c, int64_t T, int64_t max_ctx, bool contig
             const int64_t b = SkinnyFusedWorkspaceBytes(MLK_Q8_0, T, s[0], s[1]);
             if (b > p.lin_bytes) p.lin_bytes = b;
         }
+    }
+    for (const auto& g : {TileGroup{D, {QD, KD, KD}, 3}, TileGroup{QD, {D}, 1},
+                          TileGroup{D, {F, F}, 2}, TileGroup{F, {D}, 1}}) {
+        if (!TileApplies(MLK_Q8_0, T, g.in)) continue;  // (planar copies are not used there)
+        p.lin_bytes = std::max(p.lin_bytes, TileFusedPlan(T, g.in, g.rows, g.n).bytes);
     }
     if (PlanarRows(T)) {  // the same groups (and wo) on planar weights
         const int64_t groups[4][3] = {{D, QD + 2 * KD, 1}, {D, 2 * F, 1}, {F, D, 1}, {QD, D, 1}};
@@ -107,10 +116,7 @@ Plan MakePlan(const mlk_layer_config& c, int64_t T, int64_t max_ctx, bool contig
     // bf16 planes of the planar layers' x (h, attention's output, then
     // SwiGLU's output)
     const int64_t widest = std::max(D, std::max(F, QD));
-    // (many tokens: h's planes for the tiled q, k/v and gate/up launches,
-    // and the prefill attention's output planes for wo)
-    p.plane_bytes = PlanarRows(T) ? T * widest * 6
-                                  : (T > 64 && D % 32 == 0 ? T * std::max(D, QD) * 6 : 0);
+    p.plane_bytes = PlanarRows(T) ? T * widest * 6 : 0;
     p.off[10] = at;
     at += Align256(p.plane_bytes);
     p.total = at;
@@ -312,41 +318,40 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
                                SkinnyFusedApplies(w->w_gate.type, T, D));
     const bool downm = downp || (mid && w->w_down.type != kLinearF32 &&
                                  SkinnyFusedApplies(w->w_down.type, T, F));
-    // The separate q/k/v launches at consecutive positions (pos0 + T <=
-    // max_ctx <= max_seq, checked above): k and v go straight to their cache
-    // rows, which RoPE then rotates in place, so no copy launch; for many
-    // tokens k and v run as one launch where that fills the GPU without a K
-    // split (each split alone)
-    const bool kv_direct = !(qkv1 || qkvm) && contiguous;
-    float* const k_rows = kv_direct ? k_cache + (layer * max_seq + pos0) * KD : k;
-    float* const v_rows = kv_direct ? v_cache + (layer * max_seq + pos0) * KD : v;
-    const bool kv_pair = !(qkv1 || qkvm) && w->wk.type == w->wv.type &&
-                         TiledFusedApplies(w->wk.type, T, D, KD, kStreamPlain) &&
-                         Aligned(w->wk.data, 2) && Aligned(w->wv.data, 2);
-    // q alone on the tiled launch when h's planes are at hand (below)
-    const bool q_tiled = !(qkv1 || qkvm) && TiledFusedApplies(w->wq.type, T, D, QD, kStreamAdd) &&
-                         Aligned(w->wq.data, 2);
-    // Many tokens (128-row tiles, K in one pass): the same groups' epilogues
-    // in the GEMM itself, gate/up as one launch with SwiGLU, wo and down
-    // adding into x (the plain GEMM's sums, so the separate kernels' values)
-    const bool wo_add = !wop && !wo1p && TiledFusedApplies(w->wo.type, T, QD, D, kStreamAdd) &&
-                        Aligned(w->wo.data, 2);
-    const bool ffn_tiled = !ffn1 && !ffnp && !ffnm && w->w_gate.type == w->w_up.type &&
-                           TiledFusedApplies(w->w_gate.type, T, D, F, kStreamSwiGlu) &&
-                           Aligned(w->w_gate.data, 2) && Aligned(w->w_up.data, 2);
-    const bool down_tiled = !down1 && !downp && !downm &&
-                            TiledFusedApplies(w->w_down.type, T, F, D, kStreamAdd) &&
-                            Aligned(w->w_down.data, 2);
+    // more than 32 tokens: the same groups on the tiled kernel, for any one
+    // weight type per group; a group's epilogue runs in the tiles where they
+    // fill the GPU without a K split, else in the split sums' reduction
+    const auto tiled = [&](int64_t in, std::initializer_list<const mlk_linear_weight*> ws) {
+        const int t = (*ws.begin())->type;
+        if (!TileApplies(t, T, in)) return false;
+        for (const mlk_linear_weight* lw : ws) {
+            if (lw->type != t || !TileWeightAligned(t, lw->data)) return false;
+        }
+        return true;
+    };
+    const bool qkv_t = !(qkv1 || qkvm) && tiled(D, {&w->wq, &w->wk, &w->wv});
+    const bool wo_t = !wop && !wo1p && tiled(QD, {&w->wo});
+    const bool ffn_t = !ffn1 && !ffnm && tiled(D, {&w->w_gate, &w->w_up});
+    const bool down_t = !down1 && !downm && tiled(F, {&w->w_down});
+    const int64_t qkv_rows[3] = {QD, KD, KD};
+    const bool qkv_split = qkv_t && TileFusedPlan(T, D, qkv_rows, 3).splits > 1;
     // The fused q/k/v launches also rotate q and k (normal-layout pairs) and
     // write k and v into the cache rows, in place of mlk_rope_f32 and
     // mlk_kv_write_f32; the NeoX layout keeps the separate launches.
-    const bool rope_fused = (qkvm || qkv1p || (qkv1 && StreamRopeFits(D, c.head_dim))) &&
+    const bool rope_fused = (qkvm || qkv_split || qkv1p ||
+                             (qkv1 && StreamRopeFits(D, c.head_dim))) &&
                             c.rope_type == MLK_ROPE_NORMAL && c.head_dim % 2 == 0 &&
                             c.head_dim <= 2 * kRopePairs;
     if (rope_fused && positions == nullptr && (pos0 < 0 || pos0 + T > max_seq)) {
         return Fail(MLK_ERR_RANGE, "%s: positions %d..%lld out of range [0, %lld)", fn, pos0,
                     static_cast<long long>(pos0 + T - 1), static_cast<long long>(max_seq));
     }
+    // q/k/v not rotated by their launch, at consecutive positions (pos0 + T <=
+    // max_ctx <= max_seq, checked above): k and v go straight to their cache
+    // rows, which RoPE then rotates in place, so no copy launch
+    const bool kv_direct = !(qkv1 || qkvm) && !rope_fused && contiguous;
+    float* const k_rows = kv_direct ? k_cache + (layer * max_seq + pos0) * KD : k;
+    float* const v_rows = kv_direct ? v_cache + (layer * max_seq + pos0) * KD : v;
     // one token: each norm folded into the streaming GEMV that reads its
     // output (the same sums in the same order), where the norm kernel's
     // block shape allows it; the ffn norm's residual x + proj then goes to
@@ -364,17 +369,17 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
     const uint32_t* h_planes = nullptr;
     if (attn_fold) {
         // in the q/k/v launch below
-    } else if ((qkvp || q_tiled || kv_pair) && planes != nullptr &&
+    } else if (qkvp && planes != nullptr &&
                NormPlanesApplies(x, nullptr, w->attention_norm, h, D)) {
         MLK_TRY(AddRmsNormPlanes(x, nullptr, w->attention_norm, h, planes, T, D, eps, hs));
         h_planes = planes;
     } else {
         MLK_TRY(mlk_rmsnorm_f32(x, w->attention_norm, h, T, D, eps, stream));
     }
-    if (qkv1 || qkvm) {
+    if (qkv1 || qkvm || qkv_t) {
         const int64_t slot = KD;
-        float* ky = rope_fused ? k_cache + layer * max_seq * slot : k;
-        float* vy = rope_fused ? v_cache + layer * max_seq * slot : v;
+        float* ky = rope_fused ? k_cache + layer * max_seq * slot : k_rows;
+        float* vy = rope_fused ? v_cache + layer * max_seq * slot : v_rows;
         StreamArgs a{};
         const bool pl = qkvp || qkv1p;
         a.seg[0] = pl ? PlanarSeg(w->wq, q, QD) : Seg(w->wq, q, QD);
@@ -393,30 +398,15 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
                           : LinearRowStream(w->wq.type, h, D, a, mode, hs));
         } else if (qkvp) {
             MLK_TRY(LinearPlanarFused(w->wq.type, h, T, D, a, mode, lin_ws, lin_b, hs, h_planes));
+        } else if (qkv_t) {
+            MLK_TRY(LinearTileFused(w->wq.type, h, T, D, a, mode, lin_ws, lin_b, hs));
         } else {
             MLK_TRY(LinearSkinnyFused(w->wq.type, h, T, D, a, mode, lin_ws, lin_b, hs));
         }
     } else {
-        if (q_tiled && h_planes != nullptr) {  // h's planes instead of splitting h per tile
-            StreamArgs a{};
-            a.seg[0] = Seg(w->wq, q, QD);
-            a.n_seg = 1;
-            a.x_planes = h_planes;
-            MLK_TRY(LinearTiledFused(w->wq.type, h, T, D, a, kStreamPlain, hs));
-        } else {
-            MLK_TRY(Linear(w->wq, h, q, T, D, QD, lin_ws, lin_b, stream));
-        }
-        if (kv_pair) {
-            StreamArgs a{};
-            a.seg[0] = Seg(w->wk, k_rows, KD);
-            a.seg[1] = Seg(w->wv, v_rows, KD);
-            a.n_seg = 2;
-            a.x_planes = h_planes;
-            MLK_TRY(LinearTiledFused(w->wk.type, h, T, D, a, kStreamPlain, hs));
-        } else {
-            MLK_TRY(Linear(w->wk, h, k_rows, T, D, KD, lin_ws, lin_b, stream));
-            MLK_TRY(Linear(w->wv, h, v_rows, T, D, KD, lin_ws, lin_b, stream));
-        }
+        MLK_TRY(Linear(w->wq, h, q, T, D, QD, lin_ws, lin_b, stream));
+        MLK_TRY(Linear(w->wk, h, k_rows, T, D, KD, lin_ws, lin_b, stream));
+        MLK_TRY(Linear(w->wv, h, v_rows, T, D, KD, lin_ws, lin_b, stream));
     }
     if (!rope_fused) {
         MLK_TRY(mlk_rope_f32(q, k_rows, T, c.n_heads, c.n_kv_heads, c.head_dim, QD, KD, positions,
@@ -433,25 +423,39 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
     MLK_TRY(AttentionDecode(q, QD, k_cache, v_cache, n_layers, max_seq, c.n_heads, c.n_kv_heads,
                             c.head_dim, layer, positions, pos0, T, max_ctx, a, att_ws,
                             static_cast<size_t>(p.att_bytes), err, stream,
-                            (wop || (wo_add && TiledTakesPlanes(T, D))) && QD % 32 == 0
-                                ? planes
-                                : nullptr,
+                            wop && QD % 32 == 0 ? planes : nullptr,
                             &a_planes));
     h_planes = nullptr;
     const bool wo_norm = wop && ffnp && planes != nullptr && lin_ws != nullptr &&
                          NormPlanesApplies(x, static_cast<const float*>(lin_ws), w->ffn_norm, h,
                                            D) &&
                          (w->wo.bias == nullptr || Aligned(w->wo.bias, 16));
-    if (wo_norm) {
+    // the tiled wo's partial sums likewise (no planes)
+    const bool wo_t_norm = wo_t && lin_ws != nullptr && TileFusedPlan(T, QD, &D, 1).splits > 1 &&
+                           NormPlanesApplies(x, static_cast<const float*>(lin_ws), w->ffn_norm, h,
+                                             D) &&
+                           (w->wo.bias == nullptr || Aligned(w->wo.bias, 16));
+    if (wo_norm || wo_t_norm) {
         // wo's split-K partial sums reduced by the residual add + RMSNorm,
-        // which also writes h's planes for gate/up
+        // which also writes h's planes for a planar gate/up
         float* partial = nullptr;
         int splits = 1;
-        MLK_TRY(LinearPlanarPartials(w->wo.type, a, w->wo.planar, T, QD, D, lin_ws, lin_b, hs,
-                                     a_planes ? planes : nullptr, &partial, &splits));
-        MLK_TRY(AddRmsNormPlanes(x, partial, w->ffn_norm, h, planes, T, D, eps, hs, splits,
-                                 w->wo.bias));
-        h_planes = planes;
+        if (wo_norm) {
+            MLK_TRY(LinearPlanarPartials(w->wo.type, a, w->wo.planar, T, QD, D, lin_ws, lin_b, hs,
+                                         a_planes ? planes : nullptr, &partial, &splits));
+        } else {
+            MLK_TRY(LinearTilePartials(w->wo.type, a, w->wo.data, T, QD, D, lin_ws, lin_b, hs,
+                                       &partial, &splits));
+        }
+        MLK_TRY(AddRmsNormPlanes(x, partial, w->ffn_norm, h, wo_norm ? planes : nullptr, T, D, eps,
+                                 hs, splits, w->wo.bias));
+        if (wo_norm) h_planes = planes;
+    } else if (wo_t) {  // x += a Wo^T
+        StreamArgs sa{};
+        sa.seg[0] = Seg(w->wo, x, D, x);
+        sa.n_seg = 1;
+        MLK_TRY(LinearTileFused(w->wo.type, a, T, QD, sa, kStreamAdd, lin_ws, lin_b, hs));
+        MLK_TRY(mlk_rmsnorm_f32(x, w->ffn_norm, h, T, D, eps, stream));
     } else {
         if (wop) {
             MLK_TRY(LinearPlanar(w->wo.type, a, w->wo.planar, w->wo.bias, proj, T, QD, D, lin_ws,
@@ -461,24 +465,10 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
             sa.seg[0] = PlanarSeg(w->wo, proj, D);
             sa.n_seg = 1;
             MLK_TRY(LinearRowPlanar(w->wo.type, a, QD, sa, kStreamPlain, hs));
-        } else if (wo_add) {
-            StreamArgs sa{};
-            sa.seg[0] = Seg(w->wo, x, D, x);
-            sa.n_seg = 1;
-            sa.x_planes = a_planes ? planes : nullptr;  // written by the prefill attention
-            MLK_TRY(LinearTiledFused(w->wo.type, a, T, QD, sa, kStreamAdd, hs));
         } else {
             MLK_TRY(Linear(w->wo, a, proj, T, QD, D, lin_ws, lin_b, stream));
         }
-        if (wo_add && ffn_tiled && planes != nullptr &&
-            NormPlanesApplies(x, nullptr, w->ffn_norm, h, D)) {
-            // x already holds x + proj; h's planes for the gate/up launch
-            MLK_TRY(AddRmsNormPlanes(x, nullptr, w->ffn_norm, h, planes, T, D, eps, hs));
-            h_planes = planes;
-        } else if (wo_add) {  // x already holds x + proj
-            MLK_TRY(mlk_rmsnorm_f32(x, w->ffn_norm, h, T, D, eps, stream));
-        } else if ((ffnp || ffn_tiled) && planes != nullptr &&
-                   NormPlanesApplies(x, proj, w->ffn_norm, h, D)) {
+        if (ffnp && planes != nullptr && NormPlanesApplies(x, proj, w->ffn_norm, h, D)) {
             MLK_TRY(AddRmsNormPlanes(x, proj, w->ffn_norm, h, planes, T, D, eps, hs));
             h_planes = planes;
         } else if (!ffn_fold) {
@@ -515,13 +505,12 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
         a.seg[1] = Seg(w->w_up, gate, F);
         a.n_seg = 2;
         MLK_TRY(LinearSkinnyFused(w->w_gate.type, h, T, D, a, kStreamSwiGlu, lin_ws, lin_b, hs));
-    } else if (ffn_tiled) {
+    } else if (ffn_t) {
         StreamArgs a{};
         a.seg[0] = Seg(w->w_gate, gate, F);
         a.seg[1] = Seg(w->w_up, gate, F);
         a.n_seg = 2;
-        a.x_planes = h_planes;
-        MLK_TRY(LinearTiledFused(w->w_gate.type, h, T, D, a, kStreamSwiGlu, hs));
+        MLK_TRY(LinearTileFused(w->w_gate.type, h, T, D, a, kStreamSwiGlu, lin_ws, lin_b, hs));
     } else {
         MLK_TRY(Linear(w->w_gate, h, gate, T, D, F, lin_ws, lin_b, stream));
         MLK_TRY(Linear(w->w_up, h, up, T, D, F, lin_ws, lin_b, stream));
@@ -545,11 +534,11 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
         a.seg[0] = Seg(w->w_down, x, D, x);
         a.n_seg = 1;
         MLK_TRY(LinearSkinnyFused(w->w_down.type, gate, T, F, a, kStreamAdd, lin_ws, lin_b, hs));
-    } else if (down_tiled) {
+    } else if (down_t) {
         StreamArgs a{};
         a.seg[0] = Seg(w->w_down, x, D, x);
         a.n_seg = 1;
-        MLK_TRY(LinearTiledFused(w->w_down.type, gate, T, F, a, kStreamAdd, hs));
+        MLK_TRY(LinearTileFused(w->w_down.type, gate, T, F, a, kStreamAdd, lin_ws, lin_b, hs));
     } else {
         MLK_TRY(Linear(w->w_down, gate, proj, T, F, D, lin_ws, lin_b, stream));
         MLK_TRY(mlk_add_f32(x, proj, x, T * D, stream));

@@ -1,5 +1,7 @@
-// mlk_gemm.hip -- prefill-shaped linear layers on the matrix cores:
-// y[T, O] = x[T, K] W[O, K]^T (+ bias), W fp32 or Q8_0 / Q4_0 / Q4_1 blocks.
+// mlk_gemm.hip -- linear layers of several token rows on the matrix cores:
+// y[T, O] = x[T, K] W[O, K]^T (+ bias), W fp32 or Q8_0 / Q4_0 / Q4_1 blocks:
+// up to 32 rows, and the shapes of more rows that mlk_tile.hip does not take
+// (K not a multiple of 32, or below 256).
 //
 // Semantics are those of the GEMV kernels (mlk_linear.hip; the reference's
 // LinearQ80/Q40/Q41, src/quant.cc:393-463, and cublasSgemm for F32,
@@ -371,358 +373,6 @@ __global__ __launch_bounds__(kGemmThreads) void GemmMfma(const float* __restrict
             for (int r = 0; r < 4; ++r) {
                 const int64_t row = m0 + wm * (BM / 2) + 16 * i + 4 * kq + r;
                 if (row < T) out[row * O + col] = acc[i][j][r] + b;
-            }
-        }
-    }
-}
-
-// ------------------------------------------------ tiles on bf16 piece products
-// The tiled GEMM for Q8_0 / Q4_0 weights (block or planar layout) with every
-// product exact, as in GemmPlanar below: a code is a small integer, exact in
-// bf16, and x is the exact sum of three bf16 pieces, so for each block
-//   S = sum_i code_i x_i  (3 v_mfma_f32_16x16x32_bf16, fp32 sums only),
-//   acc += d * S.
-// Same tiling and split-K protocol as GemmMfma (128 token rows x 128
-// outputs, one 32-input block per stage, wave w: rows (w / 2) * 64, outputs
-// (w % 2) * 64, 4 x 4 MFMA tiles), 8x less matrix-core time per stage.  The
-// thread that loads an x float4 splits it into pieces once per stage; x
-// planes are [piece][128 rows][32 bf16] with the 16-byte group g of row r
-// at g ^ ((r / 2) % 4), and W codes [128 rows][32 bf16 + 8] (80-byte rows),
-// so the operand reads of 8 lanes meet 8 distinct bank quads.  Two stage
-// buffers, 69 KB: two workgroups per compute unit.  NW = 8 waves take 256
-// outputs per tile (90 KB, one workgroup per unit): each x split then
-// serves twice the outputs, which halves the split work per product, the
-// stage's largest VALU cost.
-typedef __bf16 bf16x8g __attribute__((ext_vector_type(8)));
-constexpr int kPcWRow = 20;  // W code row, dwords
-
-template <int BNT>
-struct __align__(16) PiecesSmem {
-    uint32_t x[2][3 * 128 * 16];
-    uint32_t w[2][BNT * kPcWRow];
-    float d[2][BNT];
-};
-
-// The pieces of 4 floats, two per dword: o[0] high, o[1] middle, o[2] low.
-// Finite values: mask and subtract; a wave with any inf or NaN takes
-// SplitBf's form (the value whole in the high piece), so products with them
-// are what fp32 products would be.  The low pieces of finite values are
-// finite and below 2^-14 of them, so their sum is NaN exactly when some
-// value is inf or NaN (inf - inf, NaN propagating): one test for four.
-__device__ inline void PiecesOf4(float4 v, uint2 (&o)[3]) {
-    const float x[4] = {v.x, v.y, v.z, v.w};
-    uint32_t h[4], m[4], l[4];
-    float lf[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const uint32_t u = __float_as_uint(x[i]);
-        const float r = x[i] - __uint_as_float(u & 0xFFFF0000u);
-        h[i] = u;
-        m[i] = __float_as_uint(r);
-        lf[i] = r - __uint_as_float(m[i] & 0xFFFF0000u);
-        l[i] = __float_as_uint(lf[i]);
-    }
-    const float chk = (lf[0] + lf[1]) + (lf[2] + lf[3]);
-    if (__builtin_amdgcn_ballot_w64(chk != chk) != 0) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            float p[3];
-            SplitBf(x[i], p);
-            h[i] = __float_as_uint(p[0]);
-            m[i] = __float_as_uint(p[1]);
-            l[i] = __float_as_uint(p[2]);
-        }
-    }
-    o[0] = make_uint2(__builtin_amdgcn_perm(h[1], h[0], 0x07060302u),
-                      __builtin_amdgcn_perm(h[3], h[2], 0x07060302u));
-    o[1] = make_uint2(__builtin_amdgcn_perm(m[1], m[0], 0x07060302u),
-                      __builtin_amdgcn_perm(m[3], m[2], 0x07060302u));
-    o[2] = make_uint2(__builtin_amdgcn_perm(l[1], l[0], 0x07060302u),
-                      __builtin_amdgcn_perm(l[3], l[2], 0x07060302u));
-}
-
-// The 16 signed codes a weight tile thread holds (inputs 16h .. 16h + 15 of
-// its row's block), as the tiles' Store decodes them; block-layout Q4_0
-// codes come as 16 x (nibble - 8) (CodeScale<WT>() undoes the 16 in the
-// scale, exactly): each dword's nibbles of half h, XOR 8, moved to the high
-// half of their bytes are those values as signed bytes, with no per-code
-// select on h.
-template <int WT>
-__device__ constexpr float CodeScale() { return WT == MLK_Q4_0 ? 0.0625f : 1.0f; }
-
-template <int WT>
-__device__ inline void TileCodes(const WTile<WT>& t, int32_t (&c)[16]) {
-    const int h = threadIdx.x & 1;
-    uint32_t sb[4];
-    if constexpr (WT == MLK_Q4_0) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) sb[j] = (((t.q[j] >> (4 * h)) & 0x0F0F0F0Fu) ^ 0x08080808u) << 4;
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        if constexpr (WT == MLK_Q8_0 || WT == kWPlanarQ8) {
-            c[i] = static_cast<int32_t>(t.q[i / 4] << (24 - 8 * (i % 4))) >> 24;
-        } else if constexpr (WT == MLK_Q4_0) {
-            c[i] = static_cast<int32_t>(sb[i / 4] << (24 - 8 * (i % 4))) >> 24;
-        } else {  // planar Q4_0: input 8g + e is nibble e (low half of byte e, then high)
-            const int e8 = i % 8;
-            const int sh = e8 < 4 ? 8 * e8 : 8 * (e8 - 4) + 4;
-            c[i] = static_cast<int32_t>(t.q[i / 8] << (28 - sh)) >> 28;
-        }
-    }
-}
-
-// Epilogues of GemmPieces (one K pass, no partial sums for the last two):
-//   kPcStore   y = sum + bias, or the split's partial sums;
-//   kPcAdd     y = y + (sum + bias), the residual add of the layer;
-//   kPcSwiGlu  gate and up in one tile (NW = 8): W rows n0 .. n0 + 127 of
-//              w (gate, waves with wn 0, 1) and of w2 (up, wn 2, 3); the gate
-//              waves hand their sums + bias through LDS to the up waves that
-//              hold the same outputs, which store SwiGlu(gate, up + bias2).
-//   kPcPair    two matrices of O rows each in one launch (the layer's k and
-//              v): the first half of the tiles along the outputs takes w,
-//              bias and y, the second w2, bias2 and y2; stored as kPcStore.
-// Each output's sum is the same as kPcStore's, so every epilogue gives the
-// separate kernels' values (mlk_add_f32, mlk_swiglu_f32) bit for bit.
-enum PiecesEpi { kPcStore = 0, kPcAdd = 1, kPcSwiGlu = 2, kPcPair = 3 };
-
-typedef uint32_t u32x4p __attribute__((ext_vector_type(4)));
-
-// kXP: x comes already split, as the planes StorePlanes writes ([K / 32
-// blocks][3 pieces][T rows][16 dwords], the pieces PiecesOf4 makes, bit for
-// bit, for every value): each stage copies 3 x 128 rows x 4 groups of 8
-// inputs (16 B) into the swizzled LDS layout, with no split in the loop
-// (the split was 7-8.5% of the linears' time at Llama-3-8B's T = 4096).
-template <int WT, int NW, int EPI = kPcStore, bool kXP = false>
-__global__ __launch_bounds__(64 * NW) void GemmPieces(const float* __restrict__ x,
-                                                           const uint8_t* __restrict__ w,
-                                                           const float* __restrict__ bias,
-                                                           float* __restrict__ y, int64_t T,
-                                                           int64_t K, int64_t O,
-                                                           int64_t row_bytes, int tiles_m,
-                                                           int tiles, int64_t per_split,
-                                                           float* __restrict__ partial,
-                                                           const uint8_t* __restrict__ w2,
-                                                           const float* __restrict__ bias2,
-                                                           float* __restrict__ y2,
-                                                           const uint32_t* __restrict__ xp) {
-    constexpr int BM = 128;
-    constexpr int kThreads = 64 * NW;
-    constexpr int BNT = 32 * NW;               // W rows per tile
-    constexpr int kXN = BM * kBK / 4 / kThreads;  // x float4s per thread and stage
-    constexpr int kXPN = 3 * BM * 4 / kThreads;   // kXP: 16-byte plane groups per thread and stage
-    constexpr bool kDual = EPI == kPcSwiGlu;
-    static_assert(!kDual || NW == 8, "gate / up tiles take 8 waves");
-    __shared__ PiecesSmem<BNT> sm;
-    const int tile = static_cast<int>(blockIdx.x) % tiles;
-    const int sp = static_cast<int>(blockIdx.x) / tiles;
-    const int tm = tile % tiles_m;
-    const int tn = tile / tiles_m;
-    const int64_t m0 = static_cast<int64_t>(tm) * BM;
-    // kPcPair: the tile's matrix (the same for the whole workgroup)
-    const int half_n = tiles / tiles_m / 2;
-    const bool wg_second = EPI == kPcPair && tn >= half_n;
-    const int64_t n0 = static_cast<int64_t>(wg_second ? tn - half_n : tn) * (kDual ? BNT / 2 : BNT);
-    // the W rows this thread loads: gate rows n0 .. for the tile's first
-    // half, up rows n0 .. (from w2) for the second when kDual
-    const bool t_second = kDual && static_cast<int>(threadIdx.x >> 1) >= BNT / 2;
-    const uint8_t* const wsrc = t_second || wg_second ? w2 : w;
-    const int64_t n0w = t_second ? n0 - BNT / 2 : n0;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
-    const int wm = wave & 1, wn = wave >> 1;  // 64 token rows x 64 outputs per wave
-    const int i16 = lane & 15, kq = lane >> 4;
-
-    f32x4 acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-
-    const int64_t all_stages = (K + kBK - 1) / kBK;
-    const int64_t s0 = sp * per_split;
-    const int64_t s1 = s0 + per_split < all_stages ? s0 + per_split : all_stages;
-    // x: thread tid holds float4 tid + kThreads i of the [128][32] stage, 8
-    // per row.  Rows past T read row 0 and W rows past O their tile's row 0,
-    // unmasked: the outputs they meet are never stored (K is a multiple of
-    // 256, so no stage reads past K).
-    // Stages are requested two ahead: registers A / B alternate, so the
-    // stage stored at the end of stage s was requested at the start of
-    // stage s - 1 and is in registers by then (requested one ahead, the
-    // scheduler moved its split next to its request and every stage waited
-    // out the load latency).
-    using XRegs = typename std::conditional<kXP, u32x4p[kXPN], float4[kXN]>::type;
-    auto load_x = [&](int64_t k0, XRegs& xv) {
-        if constexpr (kXP) {
-            // group idx: piece idx / 512, row (idx / 4) % 128, inputs 8 (idx % 4) ..
-            const uint32_t* blk = xp + (k0 / kBK) * 3 * T * 16;
-#pragma unroll
-            for (int i = 0; i < kXPN; ++i) {
-                const int idx = static_cast<int>(threadIdx.x) + kThreads * i;
-                const int64_t r = m0 + ((idx >> 2) & (BM - 1));
-                xv[i] = *reinterpret_cast<const u32x4p*>(
-                    blk + ((idx >> 9) * T + (r < T ? r : 0)) * 16 + 4 * (idx & 3));
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < kXN; ++i) {
-                const int idx = static_cast<int>(threadIdx.x) + kThreads * i;
-                const int64_t r = m0 + (idx >> 3);
-                const int64_t c = k0 + 4 * (idx & 7);
-                xv[i] = *reinterpret_cast<const float4*>(x + (r < T ? r * K + c : c));
-            }
-        }
-    };
-    // one stage into LDS buffer b: x pieces, W codes as bf16, scales
-    auto store = [&](int b, const XRegs& xv, const WTile<WT>& wt) {
-        if constexpr (kXP) {
-#pragma unroll
-            for (int i = 0; i < kXPN; ++i) {
-                const int idx = static_cast<int>(threadIdx.x) + kThreads * i;
-                const int r = (idx >> 2) & (BM - 1);
-                const int at = (idx >> 9) * 128 * 16 + r * 16 + (((idx & 3) ^ ((r >> 1) & 3)) << 2);
-                *reinterpret_cast<u32x4p*>(&sm.x[b][at]) = xv[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < kXN; ++i) {
-                const int idx = static_cast<int>(threadIdx.x) + kThreads * i;
-                const int r = idx >> 3, c8 = idx & 7;
-                uint2 pc[3];
-                PiecesOf4(xv[i], pc);
-                const int at = r * 16 + (((c8 >> 1) ^ ((r >> 1) & 3)) << 2) + 2 * (c8 & 1);
-#pragma unroll
-                for (int p = 0; p < 3; ++p) {
-                    *reinterpret_cast<uint2*>(&sm.x[b][p * 128 * 16 + at]) = pc[p];
-                }
-            }
-        }
-        int32_t c[16];
-        TileCodes<WT>(wt, c);
-        uint32_t pk[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pk[i] = PackBf(static_cast<float>(c[2 * i]), static_cast<float>(c[2 * i + 1]));
-        const int row = threadIdx.x >> 1, h = threadIdx.x & 1;
-        uint4* dst = reinterpret_cast<uint4*>(&sm.w[b][row * kPcWRow + 8 * h]);
-        dst[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
-        dst[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
-        if (h == 0) sm.d[b][row] = HalfHw(wt.d & 0xFFFFu) * CodeScale<WT>();
-    };
-    // stage s in LDS buffer (s - s0) & 1, stage s + 1 in registers `held`;
-    // stage s + 2 requested into `next` (past the last stage: the last again,
-    // never stored where it is read)
-    auto step = [&](int64_t s, const XRegs& held_x, const WTile<WT>& held_w, XRegs& next_x,
-                    WTile<WT>& next_w) {
-        const int buf = static_cast<int>((s - s0) & 1);
-        const int64_t k2 = (s + 2 < s1 ? s + 2 : s1 - 1) * kBK;
-        load_x(k2, next_x);
-        next_w.Load(wsrc, O, K, row_bytes, n0w, k2);
-        __builtin_amdgcn_sched_barrier(0);
-        bf16x8g b[4];
-        float dj[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = wn * 64 + 16 * j + i16;
-            b[j] = *reinterpret_cast<const bf16x8g*>(&sm.w[buf][row * kPcWRow + 4 * kq]);
-            dj[j] = sm.d[buf][row];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int r = wm * 64 + 16 * i + i16;
-            const int at = r * 16 + ((kq ^ ((r >> 1) & 3)) << 2);
-            bf16x8g a[3];
-#pragma unroll
-            for (int p = 0; p < 3; ++p) a[p] = *reinterpret_cast<const bf16x8g*>(&sm.x[buf][p * 128 * 16 + at]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                f32x4 S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[2], b[j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1], b[j], S, 0, 0, 0);
-                S = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[j], S, 0, 0, 0);
-#pragma unroll
-                for (int r4 = 0; r4 < 4; ++r4) acc[i][j][r4] += dj[j] * S[r4];
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        store(buf ^ 1, held_x, held_w);
-        __syncthreads();
-    };
-    XRegs xa, xb;
-    WTile<WT> wa, wb;
-    load_x(s0 * kBK, xa);
-    wa.Load(wsrc, O, K, row_bytes, n0w, s0 * kBK);
-    {
-        const int64_t k1 = (s0 + 1 < s1 ? s0 + 1 : s0) * kBK;
-        load_x(k1, xb);
-        wb.Load(wsrc, O, K, row_bytes, n0w, k1);
-    }
-    store(0, xa, wa);
-    __syncthreads();
-    for (int64_t s = s0; s < s1; s += 2) {
-        step(s, xb, wb, xa, wa);
-        if (s + 1 < s1) step(s + 1, xa, wa, xb, wb);
-    }
-
-    if constexpr (kDual) {
-        // The stage buffers are free (the last stage's reads are behind the
-        // loop's last barrier).  Gate wave (wm, wn) and up wave (wm, wn + 2)
-        // hold the same outputs in the same registers, so lane l of one
-        // hands lane l of the other its 64 sums, 16 float4s at a stride of
-        // 64 lanes (1 KB per instruction, no bank conflicts).
-        static_assert(sizeof(PiecesSmem<BNT>) >= 4 * 16 * 64 * sizeof(float4),
-                      "the gate sums fit the stage buffers");
-        float4* const xch = reinterpret_cast<float4*>(&sm) + (wm * 2 + (wn & 1)) * 16 * 64 + lane;
-        if (wn < 2) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int64_t col = n0 + wn * 64 + 16 * j + i16;
-                const float bg = bias != nullptr && col < O ? bias[col] : 0.0f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    xch[(4 * i + j) * 64] = make_float4(acc[i][j][0] + bg, acc[i][j][1] + bg,
-                                                        acc[i][j][2] + bg, acc[i][j][3] + bg);
-                }
-            }
-        }
-        __syncthreads();
-        if (wn >= 2) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int64_t col = n0 + (wn - 2) * 64 + 16 * j + i16;
-                if (col >= O) continue;
-                const float bu = bias2 != nullptr ? bias2[col] : 0.0f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float4 g4 = xch[(4 * i + j) * 64];
-                    const float g[4] = {g4.x, g4.y, g4.z, g4.w};
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int64_t row = m0 + wm * 64 + 16 * i + 4 * kq + r;
-                        if (row < T) y[row * O + col] = SwiGluF(g[r], acc[i][j][r] + bu);
-                    }
-                }
-            }
-        }
-        return;
-    }
-    float* out = partial != nullptr ? partial + sp * T * O : (wg_second ? y2 : y);
-    const float* add = partial != nullptr ? nullptr : (wg_second ? bias2 : bias);
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int64_t col = n0 + wn * 64 + 16 * j + i16;
-        if (col >= O) continue;
-        const float bb = add != nullptr ? add[col] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int64_t row = m0 + wm * 64 + 16 * i + 4 * kq + r;
-                if (row >= T) continue;
-                if constexpr (EPI == kPcAdd) {
-                    out[row * O + col] = out[row * O + col] + (acc[i][j][r] + bb);
-                } else {
-                    out[row * O + col] = acc[i][j][r] + bb;
-                }
             }
         }
     }
@@ -1631,86 +1281,10 @@ mlk_status LaunchSkinny(int wt, const float* x, const SkinnyArgs& a, int64_t T, 
     return CheckLaunch("GemmSkinny");
 }
 
-// false: no kernel of this epilogue for wt (the fused epilogues are built
-// for block-layout Q8_0 / Q4_0 only; x from planes (xp) for them too, with
-// 8 waves)
-template <int NW, int EPI = kPcStore>
-bool LaunchPieces(int wt, dim3 grid, hipStream_t s, const float* x, const uint8_t* w,
-                  const float* bias, float* y, int64_t T, int64_t K, int64_t O, int64_t row_bytes,
-                  int tiles_m, int tiles, int64_t per_split, float* partial,
-                  const uint8_t* w2 = nullptr, const float* bias2 = nullptr,
-                  float* y2 = nullptr, const uint32_t* xp = nullptr) {
-    const dim3 block(64 * NW);
-    if (xp != nullptr) {
-        // 8 waves only: at 4 the planes' registers leave one wave a SIMD
-        if constexpr (NW == 8) {
-            if (wt == MLK_Q8_0) {
-                hipLaunchKernelGGL((GemmPieces<MLK_Q8_0, NW, EPI, true>), grid, block, 0, s, x, w,
-                                   bias, y, T, K, O, row_bytes, tiles_m, tiles, per_split,
-                                   partial, w2, bias2, y2, xp);
-                return true;
-            }
-            if (wt == MLK_Q4_0) {
-                hipLaunchKernelGGL((GemmPieces<MLK_Q4_0, NW, EPI, true>), grid, block, 0, s, x, w,
-                                   bias, y, T, K, O, row_bytes, tiles_m, tiles, per_split,
-                                   partial, w2, bias2, y2, xp);
-                return true;
-            }
-        }
-        return false;
-    }
-    switch (wt) {
-        case MLK_Q8_0:
-            hipLaunchKernelGGL((GemmPieces<MLK_Q8_0, NW, EPI>), grid, block, 0, s, x, w, bias, y,
-                               T, K, O, row_bytes, tiles_m, tiles, per_split, partial, w2, bias2,
-                               y2, nullptr);
-            return true;
-        case MLK_Q4_0:
-            hipLaunchKernelGGL((GemmPieces<MLK_Q4_0, NW, EPI>), grid, block, 0, s, x, w, bias, y,
-                               T, K, O, row_bytes, tiles_m, tiles, per_split, partial, w2, bias2,
-                               y2, nullptr);
-            return true;
-        default:
-            break;
-    }
-    if constexpr (EPI == kPcStore) {
-        if (wt == kWPlanarQ8) {
-            hipLaunchKernelGGL((GemmPieces<kWPlanarQ8, NW>), grid, block, 0, s, x, w, bias, y, T,
-                               K, O, row_bytes, tiles_m, tiles, per_split, partial, w2, bias2,
-                               y2, nullptr);
-            return true;
-        }
-        if (wt == kWPlanarQ4) {
-            hipLaunchKernelGGL((GemmPieces<kWPlanarQ4, NW>), grid, block, 0, s, x, w, bias, y, T,
-                               K, O, row_bytes, tiles_m, tiles, per_split, partial, w2, bias2,
-                               y2, nullptr);
-            return true;
-        }
-    }
-    return false;
-}
-
 template <int BM>
 void LaunchTiles(int wt, dim3 grid, hipStream_t s, const float* x, const uint8_t* w,
                  const float* bias, float* y, int64_t T, int64_t K, int64_t O, int64_t row_bytes,
                  int tiles_m, int tiles, int64_t per_split, float* partial) {
-    // 128-row tiles of Q8_0 / Q4_0 on bf16 piece products; K % 256 == 0 keeps
-    // each product's fp32 roundings (block sum, scale, K / 32 block adds)
-    // under the K of the fp32 kernel's bound
-    if (BM == 128 && K % 256 == 0 &&
-        (wt == MLK_Q8_0 || wt == MLK_Q4_0 || wt == kWPlanarQ8 || wt == kWPlanarQ4)) {
-        // 256-output tiles when they still fill two workgroups per CU and K
-        // is not split; else 128
-        const int64_t tiles8 = static_cast<int64_t>(tiles_m) * ((O + 255) / 256);
-        if (per_split >= (K + kBK - 1) / kBK && tiles8 >= 2 * static_cast<int64_t>(ComputeUnits())) {
-            LaunchPieces<8>(wt, dim3(static_cast<unsigned>(tiles8)), s, x, w, bias, y, T, K, O,
-                            row_bytes, tiles_m, static_cast<int>(tiles8), per_split, partial);
-        } else {
-            LaunchPieces<4>(wt, grid, s, x, w, bias, y, T, K, O, row_bytes, tiles_m, tiles,
-                            per_split, partial);
-        }
-        return;
-    }
     switch (wt) {
         case MLK_Q8_0:
             hipLaunchKernelGGL((GemmMfma<MLK_Q8_0, BM>), grid, dim3(kGemmThreads), 0, s, x, w,
@@ -1741,7 +1315,26 @@ void LaunchTiles(int wt, dim3 grid, hipStream_t s, const float* x, const uint8_t
 
 }  // namespace
 
+mlk_status ReduceSplits(const float* partial, int splits, const float* bias, float* y, int64_t T,
+                        int64_t O, hipStream_t s) {
+    hipLaunchKernelGGL(SplitKReduce, dim3(GridFor(T * O, kGemmThreads, 8)), dim3(kGemmThreads), 0,
+                       s, partial, splits, bias, y, T, O);
+    return CheckLaunch("SplitKReduce");
+}
+
+mlk_status ReduceSplitsFused(const float* partial, int splits, int64_t T, int64_t cols,
+                             const StreamArgs& sa, int mode, hipStream_t s) {
+    const int64_t out_cols = mode == kStreamSwiGlu    ? sa.seg[0].rows
+                             : mode == kStreamQkvRope ? (sa.seg[0].rows + sa.seg[1].rows) / 2 +
+                                                            sa.seg[2].rows
+                                                      : cols;
+    hipLaunchKernelGGL(SplitKReduceFused, dim3(GridFor(T * out_cols, kGemmThreads, 8)),
+                       dim3(kGemmThreads), 0, s, partial, splits, T, cols, sa, mode, out_cols);
+    return CheckLaunch("SplitKReduceFused");
+}
+
 int64_t GemmWorkspaceBytes(int wt, int64_t T, int64_t K, int64_t O) {
+    if (TileApplies(wt, T, K)) return TileWorkspaceBytes(T, K, O);
     const SplitPlan p = SkinnyApplies(wt, T, K) ? PlanSkinny(wt, T, K) : PlanSplits(T, K, O);
     return p.splits > 1 ? static_cast<int64_t>(p.splits) * T * O * 4 : 0;
 }
@@ -1755,6 +1348,9 @@ int64_t GemmWorkspaceBytes(int wt, int64_t T, int64_t K, int64_t O) {
 mlk_status LaunchGemm(int wt, const float* x, const void* w, const float* bias, float* y,
                       int64_t T, int64_t K, int64_t O, int64_t row_bytes, void* workspace,
                       size_t workspace_bytes, hipStream_t s) {
+    if (TileApplies(wt, T, K)) {
+        return LaunchTile(wt, x, w, bias, y, T, K, O, row_bytes, workspace, workspace_bytes, s);
+    }
     const SplitPlan sk = PlanSkinny(wt, T, K);
     const bool sk_ws = sk.splits == 1 ||
                        (workspace != nullptr && Aligned(workspace, 16) &&
@@ -1777,9 +1373,7 @@ mlk_status LaunchGemm(int wt, const float* x, const void* w, const float* bias, 
         a.y = y;
         mlk_status st = LaunchSkinny(wt, x, a, T, K, row_bytes, plan.splits, partial, s);
         if (st != MLK_OK || partial == nullptr) return st;
-        hipLaunchKernelGGL(SplitKReduce, dim3(GridFor(T * O, kGemmThreads, 8)),
-                           dim3(kGemmThreads), 0, s, partial, plan.splits, bias, y, T, O);
-        return CheckLaunch("SplitKReduce");
+        return ReduceSplits(partial, plan.splits, bias, y, T, O, s);
     }
     const int bm = TileRows(T);
     const int64_t tiles_m = (T + bm - 1) / bm;
@@ -1814,116 +1408,7 @@ mlk_status LaunchGemm(int wt, const float* x, const void* w, const float* bias, 
     }
     mlk_status st = CheckLaunch("GemmMfma");
     if (st != MLK_OK || partial == nullptr) return st;
-    hipLaunchKernelGGL(SplitKReduce, dim3(GridFor(T * O, kGemmThreads, 8)), dim3(kGemmThreads), 0,
-                       s, partial, plan.splits, bias, y, T, O);
-    return CheckLaunch("SplitKReduce");
-}
-
-bool TiledFusedApplies(int wt, int64_t T, int64_t K, int64_t O, int mode) {
-    if ((wt != MLK_Q8_0 && wt != MLK_Q4_0) || K % 256 != 0 || TileRows(T) != 128 || O <= 0) {
-        return false;
-    }
-    const int64_t tiles_m = (T + 127) / 128;
-    if (mode == kStreamPlain) {  // a pair in one pass, where that fills the GPU on its own
-        const int64_t tiles = tiles_m * 2 * ((O + 127) / 128);
-        return tiles >= 2 * static_cast<int64_t>(ComputeUnits()) && tiles <= 0x7FFFFFFF;
-    }
-    if (PlanSplits(T, K, O).splits != 1) return false;
-    if (mode == kStreamSwiGlu) {
-        const int64_t tiles = tiles_m * ((O + 127) / 128);
-        return tiles >= 2 * static_cast<int64_t>(ComputeUnits()) && tiles <= 0x7FFFFFFF;
-    }
-    return mode == kStreamAdd && tiles_m * ((O + 127) / 128) <= 0x7FFFFFFF;
-}
-
-bool TiledTakesPlanes(int64_t T, int64_t O) {
-    return ((T + 127) / 128) * ((O + 255) / 256) >= 2 * static_cast<int64_t>(ComputeUnits());
-}
-
-mlk_status LinearTiledFused(int wt, const float* x, int64_t T, int64_t K, const StreamArgs& sa,
-                            int mode, hipStream_t s) {
-    const StreamSeg& g0 = sa.seg[0];
-    const int64_t O = g0.rows;
-    const bool single = mode == kStreamPlain && sa.n_seg == 1;
-    if (!TiledFusedApplies(wt, T, K, O, single ? kStreamAdd : mode) || !Aligned(x, 16) ||
-        (sa.x_planes != nullptr && !Aligned(sa.x_planes, 16))) {
-        return Fail(MLK_ERR_INVALID, "linear (tiled, fused): unsupported shape");
-    }
-    if (single) {
-        if (g0.w == nullptr || g0.y == nullptr || !Aligned(g0.w, 2)) {
-            return Fail(MLK_ERR_INVALID, "linear (tiled, fused): bad segment");
-        }
-    } else if (mode == kStreamSwiGlu || mode == kStreamPlain) {
-        const StreamSeg& g1 = sa.seg[1];
-        if (sa.n_seg != 2 || g1.rows != O || g0.w == nullptr || g1.w == nullptr ||
-            g1.y == nullptr || (mode == kStreamPlain && g0.y == nullptr) || !Aligned(g0.w, 2) ||
-            !Aligned(g1.w, 2)) {
-            return Fail(MLK_ERR_INVALID, "linear (tiled, fused): bad segment pair");
-        }
-    } else if (sa.n_seg != 1 || g0.w == nullptr || g0.y == nullptr || g0.res != g0.y ||
-               !Aligned(g0.w, 2)) {
-        // the residual add runs in place: y = y + sum
-        return Fail(MLK_ERR_INVALID, "linear (tiled, fused): the residual must be y");
-    }
-    // the outputs are written while other workgroups still read x
-    const auto overlaps_x = [&](const float* y) {
-        return y != nullptr && y < x + T * K && x < y + T * O;
-    };
-    if (overlaps_x(g0.y) || (sa.n_seg == 2 && overlaps_x(sa.seg[1].y))) {
-        return Fail(MLK_ERR_INVALID, "linear (tiled, fused): outputs must not overlap x");
-    }
-    const int64_t row_bytes = (K / 32) * BlockBytes(wt);
-    const int64_t stages = K / kBK;
-    const int tm = static_cast<int>((T + 127) / 128);
-    bool ok = false;
-    const uint32_t* xp = sa.x_planes;
-    if (single) {
-        // the tile width LaunchTiles takes for the plain product
-        const int64_t tiles8 = static_cast<int64_t>(tm) * ((O + 255) / 256);
-        if (tiles8 >= 2 * static_cast<int64_t>(ComputeUnits())) {
-            const int tiles = static_cast<int>(tiles8);
-            ok = LaunchPieces<8>(wt, dim3(static_cast<unsigned>(tiles)), s, x, g0.w, g0.bias, g0.y,
-                                 T, K, O, row_bytes, tm, tiles, stages, nullptr, nullptr, nullptr,
-                                 nullptr, xp);
-        } else {
-            // 4-wave tiles split x themselves (no planes variant)
-            const int tiles = static_cast<int>(tm * ((O + 127) / 128));
-            ok = LaunchPieces<4>(wt, dim3(static_cast<unsigned>(tiles)), s, x, g0.w, g0.bias, g0.y,
-                                 T, K, O, row_bytes, tm, tiles, stages, nullptr);
-        }
-    } else if (mode == kStreamPlain) {
-        // 256-output tiles (TiledFusedApplies leaves at least one a CU):
-        // each x split serves twice the outputs of a 128-output tile;
-        // measured at Llama-3-8B's k / v (256 tiles) as fast as 512 tiles
-        // of 128 outputs, or slightly faster
-        const int tiles = static_cast<int>(static_cast<int64_t>(tm) * 2 * ((O + 255) / 256));
-        const StreamSeg& g1 = sa.seg[1];
-        ok = LaunchPieces<8, kPcPair>(wt, dim3(static_cast<unsigned>(tiles)), s, x, g0.w, g0.bias,
-                                      g0.y, T, K, O, row_bytes, tm, tiles, stages, nullptr, g1.w,
-                                      g1.bias, g1.y, xp);
-    } else if (mode == kStreamSwiGlu) {
-        const int tiles = static_cast<int>(tm * ((O + 127) / 128));
-        ok = LaunchPieces<8, kPcSwiGlu>(wt, dim3(static_cast<unsigned>(tiles)), s, x, g0.w,
-                                        g0.bias, sa.seg[1].y, T, K, O, row_bytes, tm, tiles,
-                                        stages, nullptr, sa.seg[1].w, sa.seg[1].bias, nullptr,
-                                        xp);
-    } else {
-        // the tile width LaunchTiles takes for the plain product
-        const int64_t tiles8 = static_cast<int64_t>(tm) * ((O + 255) / 256);
-        if (tiles8 >= 2 * static_cast<int64_t>(ComputeUnits())) {
-            const int tiles = static_cast<int>(tiles8);
-            ok = LaunchPieces<8, kPcAdd>(wt, dim3(static_cast<unsigned>(tiles)), s, x, g0.w,
-                                         g0.bias, g0.y, T, K, O, row_bytes, tm, tiles, stages,
-                                         nullptr, nullptr, nullptr, nullptr, xp);
-        } else {
-            const int tiles = static_cast<int>(tm * ((O + 127) / 128));
-            ok = LaunchPieces<4, kPcAdd>(wt, dim3(static_cast<unsigned>(tiles)), s, x, g0.w,
-                                         g0.bias, g0.y, T, K, O, row_bytes, tm, tiles, stages,
-                                         nullptr);
-        }
-    }
-    if (!ok) return Fail(MLK_ERR_INVALID, "linear (tiled, fused): weight type %d", wt);
-    return CheckLaunch("GemmPieces (fused)");
+    return ReduceSplits(partial, plan.splits, bias, y, T, O, s);
 }
 
 bool SkinnyFusedApplies(int wt, int64_t T, int64_t K) {
@@ -1973,14 +1458,7 @@ mlk_status LinearSkinnyFused(int wt, const float* x, int64_t T, int64_t K, const
     const int64_t row_bytes = (K / 32) * BlockBytes(wt);
     mlk_status st = LaunchSkinny(wt, x, a, T, K, row_bytes, plan.splits, partial, s);
     if (st != MLK_OK) return st;
-    const int64_t out_cols = mode == kStreamSwiGlu    ? sa.seg[0].rows
-                             : mode == kStreamQkvRope ? (sa.seg[0].rows + sa.seg[1].rows) / 2 +
-                                                            sa.seg[2].rows
-                                                      : cols;
-    hipLaunchKernelGGL(SplitKReduceFused, dim3(GridFor(T * out_cols, kGemmThreads, 8)),
-                       dim3(kGemmThreads), 0, s, partial, plan.splits, T, cols, sa, mode,
-                       out_cols);
-    return CheckLaunch("SplitKReduceFused");
+    return ReduceSplitsFused(partial, plan.splits, T, cols, sa, mode, s);
 }
 
 // ------------------------------------------------------- planar launches
@@ -2202,9 +1680,7 @@ mlk_status LinearPlanar(int qt, const float* x, const void* w, const float* bias
     mlk_status st = RunPlanar(qt, x, planes, a, T, K, false, workspace, workspace_bytes,
                               &splits, &partial, s);
     if (st != MLK_OK || partial == nullptr) return st;
-    hipLaunchKernelGGL(SplitKReduce, dim3(GridFor(T * O, kGemmThreads, 8)), dim3(kGemmThreads), 0,
-                       s, partial, splits, bias, y, T, O);
-    return CheckLaunch("SplitKReduce");
+    return ReduceSplits(partial, splits, bias, y, T, O, s);
 }
 
 mlk_status LinearPlanarPartials(int qt, const float* x, const void* w, int64_t T, int64_t K,
@@ -2249,14 +1725,7 @@ mlk_status LinearPlanarFused(int qt, const float* x, int64_t T, int64_t K, const
     mlk_status st = RunPlanar(qt, x, planes, a, T, K, true, workspace, workspace_bytes, &splits,
                               &partial, s);
     if (st != MLK_OK) return st;
-    const int64_t cols = a.cols;
-    const int64_t out_cols = mode == kStreamSwiGlu    ? sa.seg[0].rows
-                             : mode == kStreamQkvRope ? (sa.seg[0].rows + sa.seg[1].rows) / 2 +
-                                                            sa.seg[2].rows
-                                                      : cols;
-    hipLaunchKernelGGL(SplitKReduceFused, dim3(GridFor(T * out_cols, kGemmThreads, 8)),
-                       dim3(kGemmThreads), 0, s, partial, splits, T, cols, sa, mode, out_cols);
-    return CheckLaunch("SplitKReduceFused");
+    return ReduceSplitsFused(partial, splits, T, a.cols, sa, mode, s);
 }
 
 }  // namespace mlk

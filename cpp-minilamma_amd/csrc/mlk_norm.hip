@@ -261,11 +261,16 @@ mlk_status AddRmsNormPlanes(float* residual, const float* delta, const float* we
                             uint32_t* planes, int64_t n_rows, int64_t dim, float eps,
                             hipStream_t s, int splits, const float* dbias) {
     if (!NormPlanesApplies(residual, delta, weight, y, dim) || !Aligned(planes, 16) ||
-        (dbias != nullptr && !Aligned(dbias, 16)) || splits < 1) {
+        (dbias != nullptr && !Aligned(dbias, 16)) || splits < 1 ||
+        (planes == nullptr && delta == nullptr)) {
         return Fail(MLK_ERR_INVALID, "rmsnorm (planes): unsupported row layout");
     }
     if (delta == nullptr) {
         return Launch<false, false, true>(residual, nullptr, weight, y, n_rows, dim, eps, s, planes);
+    }
+    if (planes == nullptr) {
+        return Launch<true, true, false, true>(residual, delta, weight, y, n_rows, dim, eps, s,
+                                               nullptr, splits, dbias);
     }
     if (splits > 1 || dbias != nullptr) {
         return Launch<true, true, true, true>(residual, delta, weight, y, n_rows, dim, eps, s,

@@ -122,9 +122,6 @@ struct StreamArgs {
     // outputs also go here as bf16 planes (StorePlanes, mlk_common.h) for
     // the next planar layer; F % 32 == 0
     uint32_t* planes = nullptr;
-    // LinearTiledFused only: x already split into planes (StorePlanes
-    // layout, 16-byte aligned), read instead of x by 8-wave tiles
-    const uint32_t* x_planes = nullptr;
 };
 
 // in_features % 64 == 0 and x (16-byte aligned) fits the kernel's LDS
@@ -166,27 +163,42 @@ mlk_status LaunchGemm(int wt, const float* x, const void* w, const float* bias, 
                       int64_t T, int64_t K, int64_t O, int64_t row_bytes, void* workspace,
                       size_t workspace_bytes, hipStream_t s);
 int64_t GemmWorkspaceBytes(int wt, int64_t T, int64_t K, int64_t O);
-// The same tiled product with the layer's epilogue in one launch (no
-// workspace) for many token rows: block-layout Q8_0 / Q4_0, K % 256 == 0,
-// T > 64, O rows per matrix, and only where LaunchGemm would not split K
-// either, so each output's sum is LaunchGemm's.  kStreamAdd: one segment
-// with res == y (y = y + (sum + bias), mlk_add_f32's value).  kStreamSwiGlu:
-// gate and up segments of O rows each, seg[1].y = SwiGlu(gate, up) as
-// mlk_swiglu_f32 computes it, when the gate / up tiles fill two workgroups
-// per CU.  kStreamPlain: two matrices of O rows each (segments 0 and 1,
-// each to its own y) in one launch without a K split, when their tiles
-// together fill two workgroups per CU (where LaunchGemm would split each:
-// the sums are then the unsplit product's, LaunchGemm's without a
-// workspace); with one segment, that matrix alone, under kStreamAdd's shape
-// rule (LaunchGemm's sums).  a.x_planes, when set, holds x as StorePlanes
-// writes it and the 8-wave tiles read it instead of splitting x (the same
-// sums; 4-wave tiles still read x).  x 16-byte aligned, W 2-byte aligned.
-bool TiledFusedApplies(int wt, int64_t T, int64_t K, int64_t O, int mode);
-// A one-matrix or residual-add launch of O rows takes the 8-wave tiles,
-// which read x_planes (the pair and SwiGLU launches always do).
-bool TiledTakesPlanes(int64_t T, int64_t O);
-mlk_status LinearTiledFused(int wt, const float* x, int64_t T, int64_t K, const StreamArgs& a,
-                            int mode, hipStream_t s);
+// Partial sums [splits][T][O] added in split order, + bias, into y; and the
+// same with a fused launch's epilogue (modes and segments as for
+// LinearSkinnyFused, the segments' columns side by side, cols together).
+mlk_status ReduceSplits(const float* partial, int splits, const float* bias, float* y, int64_t T,
+                        int64_t O, hipStream_t s);
+mlk_status ReduceSplitsFused(const float* partial, int splits, int64_t T, int64_t cols,
+                             const StreamArgs& a, int mode, hipStream_t s);
+
+// Many rows on the fp16 matrix cores (mlk_tile.hip): LaunchGemm's shapes
+// with more than 32 rows, K a multiple of 32 (planar: 256) and 256 or more.
+// Alignments and workspace as LaunchGemm.
+bool TileApplies(int wt, int64_t T, int64_t K);
+int64_t TileWorkspaceBytes(int64_t T, int64_t K, int64_t O);
+mlk_status LaunchTile(int wt, const float* x, const void* w, const float* bias, float* y, int64_t T,
+                      int64_t K, int64_t O, int64_t row_bytes, void* workspace,
+                      size_t workspace_bytes, hipStream_t s);
+// Up to three fp32 or block-layout weight matrices of one type with the same
+// K in one launch, with a layer's epilogue: in the tiles when K is not split
+// (plain, residual add in place with res == y, SwiGLU), else in the
+// reduction (those and kStreamQkvRope, which needs a split).  Unsplit sums
+// are LaunchTile's.  TileFusedPlan: the K splits of such a launch and its
+// workspace (16-byte aligned; 0 bytes without a split).
+struct TileFused {
+    int splits = 1;
+    int64_t bytes = 0;
+};
+TileFused TileFusedPlan(int64_t T, int64_t K, const int64_t* rows, int n_seg);
+mlk_status LinearTileFused(int wt, const float* x, int64_t T, int64_t K, const StreamArgs& a,
+                           int mode, void* workspace, size_t workspace_bytes, hipStream_t s);
+// The launch alone, for a caller that reduces: one matrix's partial sums in
+// the workspace (TileFusedPlan says splits > 1).
+mlk_status LinearTilePartials(int wt, const float* x, const void* w, int64_t T, int64_t K,
+                              int64_t O, void* workspace, size_t workspace_bytes, hipStream_t s,
+                              float** partial, int* splits);
+// 16-byte alignment of fp32 weights, 4 for Q4_1 blocks, 2 for the others
+bool TileWeightAligned(int wt, const void* w);
 
 // Planar Q8_0 / Q4_0 weights (layout at mlk_quant_to_planar, minilamma_hip.h;
 // mlk_gemm.hip).  wt values of LaunchGemm for them:
@@ -215,7 +227,7 @@ mlk_status LinearPlanarFused(int qt, const float* x, int64_t T, int64_t K, const
 // the planar layers (StorePlanes, mlk_common.h), when NormPlanesApplies.
 // splits > 1 or dbias: delta holds a linear layer's split-K partial sums
 // ([splits][n_rows][dim]), reduced here in split order, then + dbias, as
-// SplitKReduce would.
+// SplitKReduce would; planes may then be null (not written).
 bool NormPlanesApplies(const float* residual, const float* delta, const float* weight,
                        const float* y, int64_t dim);
 // AddRmsNormVec's block for rows of dim floats (false: another kernel takes

@@ -171,8 +171,8 @@ mlk_status mlk_linear_f32(const float* x, const float* w, const float* bias, flo
 
 /* Device bytes of the optional workspace of mlk_linear_quant / mlk_linear_f32
  * for this shape on the current device (0: the call uses none).  Calls of
- * 32 rows or more run on the matrix cores in 128 x 128 output tiles; when
- * those tiles are fewer than two per compute unit, a workspace of this size
+ * 8 rows or more run on the matrix cores in output tiles; when those tiles
+ * are too few to fill the compute units, a workspace of this size
  * (16-byte aligned, not aliasing x, W or y) lets the call split K over
  * workgroups and add the partial sums in a fixed order.  Without it (NULL or
  * smaller) the call is still correct, only slower.  No counterpart in the
@@ -208,8 +208,9 @@ mlk_status mlk_quant_to_planar(int32_t quant_type, const void* blocks, int64_t r
  * matrix cores with exact products (codes are exact in bf16 and x is split
  * into three exact bf16 pieces), and need a workspace of
  * mlk_linear_planar_workspace_bytes (16-byte aligned); more rows take the
- * tiled matrix-core GEMM (from 65 rows with in_features a multiple of 256,
- * on the same exact bf16 products), with the optional workspace of
+ * tiled matrix-core GEMM (x in two fp16 pieces under a power of two per row,
+ * each value to within one unit of its fp32 last place; rows outside the
+ * pieces' range in fp32), with the optional workspace of
  * mlk_linear_workspace_bytes.  No counterpart in the reference. */
 mlk_status mlk_linear_planar(int32_t quant_type, const float* x, const void* w_planar,
                              const float* bias, float* y, int64_t rows, int64_t in_features,
@@ -360,9 +361,7 @@ typedef struct {
  * tokens attending up to max_ctx positions; consecutive_positions != 0 when
  * the call passes positions == NULL (0 on bad input).  A prompt chunk of
  * 1024 or more tokens at head_dim 128 includes the attention's pre-split
- * K/V (12 bytes per cached K and V element of a layer up to max_ctx), and
- * more than 64 tokens the bf16 planes of the normed rows (6 * n_tokens *
- * dim bytes). */
+ * K/V (12 bytes per cached K and V element of a layer up to max_ctx). */
 int64_t mlk_forward_layer_workspace_bytes(const mlk_layer_config* cfg, int64_t n_tokens,
                                           int64_t max_ctx, int32_t consecutive_positions);
 

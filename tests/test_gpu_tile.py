@@ -1,0 +1,131 @@
+"""The many-row linear kernel on fp16 pieces (csrc/mlk_tile.hip): more than 32
+rows, in_features a multiple of 32 and at least 256.
+
+Bar: every output within gamma_K * sum_k |x_k w_k| of the float64 product
+with the dequantized weights (conftest.assert_dot_close).  A product here is
+within 3 * 2^-22 of its exact value (each operand to one unit of its last of
+23 bits, the product of the two low pieces left out), 12 u; with K >= 256 and
+one fp32 rounding per 32 inputs and piece the sums stay below K u."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle as O
+from conftest import assert_dot_close, dot_exact
+
+pytestmark = pytest.mark.gpu
+
+TYPES = ("q8_0", "q4_0", "q4_1", "f32", "planar q8_0", "planar q4_0")
+SHAPES = [  # (out, in, rows): tile edges, an odd number of 32-input blocks, K splits of uneven length
+    (1, 256, 33), (127, 288, 64), (129, 320, 65), (128, 4128, 128), (255, 512, 129),
+    (257, 256, 300), (4099, 1024, 70), (12300, 256, 2050)]
+
+
+def normal(rng, shape, std=1.0):
+    return (rng.standard_normal(shape) * std).astype(np.float32)
+
+
+def run(mlk, orc, kind, x, w, bias=None, workspace="auto"):
+    """(y, the float64 weights' fp32 values)."""
+    T, K = x.shape
+    out = w.shape[0]
+    B = mlk.DeviceBuffer.from_array
+    y = mlk.DeviceBuffer.empty((T, out))
+    b = None if bias is None else B(bias)
+    if kind == "f32":
+        mlk.linear_f32(B(x), B(w), y, T, K, out, bias=b, workspace=workspace)
+        return y.download(), w
+    qt = kind.split()[-1]
+    blocks = orc.quantize(qt, w)
+    d_w = B(np.ascontiguousarray(blocks, np.uint8))
+    if kind.startswith("planar"):
+        p = mlk.DeviceBuffer(mlk.quant_planar_bytes(qt, out, K), np.uint8)
+        mlk.quant_to_planar(qt, d_w, out, K, p)
+        mlk.linear_planar(qt, B(x), p, y, T, K, out, bias=b)
+    else:
+        mlk.linear_quant(qt, B(x), d_w, y, T, K, out, bias=b, workspace=workspace)
+    return y.download(), orc.dequantize(qt, blocks, out, K)
+
+
+@pytest.mark.parametrize("kind", TYPES)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_tile_shapes(mlk, orc, kind, shape):
+    out, K, T = shape
+    if kind.startswith("planar") and K % 256:
+        pytest.skip("no planar layout")
+    rng = np.random.default_rng(out + K + T)
+    w, x, bias = normal(rng, (out, K), 0.02), normal(rng, (T, K)), normal(rng, (out,), 0.1)
+    for workspace in ("auto", None):
+        got, wd = run(mlk, orc, kind, x, w, bias, workspace)
+        ex, s = dot_exact(x, wd, bias)
+        assert_dot_close(got, ex, s, K + 1, f"{kind} {shape} workspace={workspace}")
+
+
+@pytest.mark.parametrize("kind", TYPES)
+@pytest.mark.parametrize("T", [40, 200])
+def test_tile_row_scales(mlk, orc, kind, T):
+    """Rows of every magnitude in one tile: the row's power of two brings
+    ordinary ones into fp16's range; rows that stay outside (an outlier over
+    16384 times the first inputs' mean, first inputs zero and the rest tiny,
+    beyond 2^61) are summed in fp32.  Zero rows stay zero; infinities and
+    NaNs give what the products give.  fp32 weights get the same rows."""
+    out, K = 300, 512
+    rng = np.random.default_rng(T)
+    x, w = normal(rng, (T, K)), normal(rng, (out, K), 0.02)
+
+    def spread(m):
+        m[1] = 0
+        m[2] *= 1e-12
+        m[3] *= 1e12
+        m[4] *= 1e-25
+        m[5] *= 1e25
+        m[6, 100] = 5e5
+        m[7, :64] = 0
+        m[8, :64] = 0
+        m[8] *= 1e-9
+        m[9, :64] *= 1e-4
+        m[10, :64] *= 1e4
+        m[11, ::2] = 0
+        m[12] = np.where(np.arange(K) % 37 == 0, m[12] * 1e7, m[12])
+    spread(x)
+    if kind == "f32":
+        spread(w)
+    bad = [20, 21, 22]
+    x[20, 70], x[21, 3], x[22, 500] = np.inf, np.nan, -np.inf
+    got, wd = run(mlk, orc, kind, x, w)
+    with np.errstate(invalid="ignore", over="ignore"):
+        want = x.astype(np.float64) @ wd.astype(np.float64).T
+    for t in bad:
+        np.testing.assert_array_equal(np.isnan(got[t]), np.isnan(want[t]))
+        inf = np.isinf(want[t])
+        np.testing.assert_array_equal(got[t][inf], want[t][inf])
+    ok = np.setdiff1d(np.arange(T), bad)
+    ex, s = dot_exact(x[ok], wd)
+    fits = s < 3e38  # (5e25-sized rows of both operands)
+    u = 2.0 ** -24
+    err = np.abs(got[ok].astype(np.float64) - ex)
+    lim = K * u / (1 - K * u) * s + 1e-44
+    assert (err[fits] <= lim[fits]).all(), f"{kind}: {int((err > lim)[fits].sum())} outside"
+
+
+@pytest.mark.parametrize("wt", ["q8_0", "q4_1", "f32"])
+@pytest.mark.parametrize("gaps", [False, True])
+def test_tile_layer_matches_oracle(orc, mlk, wt, gaps):
+    """A layer's fused launches with a K split (q/k/v rotated and cached in
+    the reduction, wo's sums reduced by the norm, SwiGLU and the residual add
+    in reductions): two layers over 70 tokens, consecutive and at increasing
+    positions, against the oracle's token loop."""
+    import importlib
+    fwd = importlib.import_module(mlk.__name__ + ".forward")
+    cfg = dict(vocab=200, dim=512, hidden_dim=1024, layers=2, n_heads=8, n_kv_heads=2,
+               head_dim=64, max_seq=256, rope_type=0, theta=10000.0, eps=1e-5)
+    model = O.forward_model(cfg, seed=5, weight_type=wt, biases=True)
+    T = 70
+    tokens = (np.arange(T, dtype=np.int32) * 11 + 3) % 200
+    pos = np.cumsum(np.arange(T) % 4 + 1 if gaps else np.ones(T)).astype(np.int32) - 1
+    want, _ = orc.forward_tokens(model, tokens, pos)
+    dm = fwd.DeviceModel(model)
+    x = dm.hidden(tokens, positions=pos if gaps else None)
+    got = dm.logits(x, T).download().astype(np.float64)
+    assert (np.abs(got - want) <= 1e-5 + 1e-4 * np.abs(want)).all()
