@@ -16,15 +16,16 @@ bool PrefillSupported(int32_t head_dim, const float* q, int64_t q_row_stride, co
 // slot = KV * head_dim floats per position.  Arguments already validated.
 // With a 16-byte aligned workspace of PrefillImageBytes(KV, head_dim,
 // pos0 + T) bytes (head_dim 128, T >= kPrefillImageMinTokens), K and V of
-// positions 0 .. pos0 + T - 1 are first split into bf16 piece images, one
+// positions 0 .. pos0 + T - 1 are first split into fp16 piece images, one
 // launch, which the tiles then copy instead of splitting each tile in every
 // workgroup; the sums are the same.  Otherwise no workspace is used.  Below
 // that many tokens a tile is staged by too few workgroups for the extra
-// launch to pay (Llama-3-70B heads, T = 512: 44 -> 48 us with the images;
-// T = 4096: 1569 -> 1443 us).  a_planes (16-byte aligned, H * head_dim a
+// launch to pay (Llama-3-8B heads, from position 0: 128 tokens 14.8 -> 14.1
+// us with the images, 64 tokens 10.0 -> 10.9; 389 tokens at 1500: 133 -> 96,
+// 4096 tokens 629 -> 483).  a_planes (16-byte aligned, H * head_dim a
 // multiple of 32), when set, also receives the output rows as StorePlanes
 // planes.
-constexpr int64_t kPrefillImageMinTokens = 1024;
+constexpr int64_t kPrefillImageMinTokens = 128;
 int64_t PrefillImageBytes(int32_t n_kv_heads, int32_t head_dim, int64_t n_pos);
 mlk_status LaunchPrefill(const float* q, int64_t q_row_stride, const float* kc, const float* vc,
                          int64_t slot, int32_t H, int32_t KV, int32_t head_dim, int32_t pos0,

@@ -609,6 +609,48 @@ def test_attention_tiles_dropped_pieces_within_bound(mlk):
                                pieces=True)
 
 
+@pytest.mark.parametrize("T,pos0", [(16, 64), (33, 63), (128, 37), (200, 0)])
+def test_attention_tiles_of_far_apart_magnitudes(mlk, T, pos0):
+    """The fp16 pieces' scales: 32-position tiles whose K and V differ by up to
+    2^126, one of them zero, and a zero query row; through the prefill kernel
+    (T below and from the images' 128 tokens, ragged last blocks) and the
+    shared decode tiles.  Each V and p is within 2^-39 of its tile's largest
+    (of 1), on top of its own 2^-23: at most 2^-38 (n + 1) M more than the
+    tiles' bound, M the KV head's largest |V| up to the end of the tile of the
+    token block's last position."""
+    rng = np.random.default_rng(T + pos0)
+    H, KV, hd = 8, 2, 128
+    S = pos0 + T
+    kc, vc = random_cache(rng, 2, S, KV, hd)
+    for tile in range((S + 31) // 32):
+        rows = slice(32 * tile, 32 * tile + 32)
+        kc[:, rows] *= np.float32(2.0 ** -(30 * (tile % 3)))
+        vc[:, rows] *= np.float32(0.0 if tile == 2 else 2.0 ** (63 - 21 * (tile % 7)))
+    cache = Cache(mlk, kc, vc)
+    q = rng.standard_normal((T, H, hd)).astype(np.float32)
+    q[T // 2] = 0.0
+    ex, pav, dmax, n = prefill_exact(q, kc, vc, 1, pos0)
+
+    def more(last, tokens):
+        m = np.abs(vc[1, :last // 32 * 32 + 32]).max(axis=(0, 2)).astype(np.float64)
+        return 2.0 ** -38 * (tokens + 1) * np.repeat(m, H // KV)[:, None]
+
+    def check(got, t, last, what):
+        bound = (2 * dmax[t][:, None] + (n[t] + 22) * U) * pav[t] + more(last, n[t]) + 1e-30
+        assert np.isfinite(got).all(), f"{what}: non-finite output"
+        err = np.abs(got.astype(np.float64) - ex[t])
+        assert (err <= bound).all(), f"{what} token {t}: worst {float((err / bound).max()):.3g}"
+
+    for images in (False, True):
+        got = run_prefill(mlk, cache, q, 1, pos0, images=images)
+        for t in range(T):
+            check(got[t], t, min(pos0 + t // 16 * 16 + 15, S - 1), f"images {images}")
+    pos = np.sort(rng.choice(np.arange(pos0, S), 16, replace=False)).astype(np.int32)
+    got = cache.attend(q[pos - pos0], 1, pos)
+    for i, p in enumerate(pos):
+        check(got[i], p - pos0, S - 1, "decode tiles")
+
+
 def test_attention_prefill_rejects(mlk):
     kc = mlk.DeviceBuffer.empty((2, 64, 2, 128))
     vc = mlk.DeviceBuffer.empty((2, 64, 2, 128))
