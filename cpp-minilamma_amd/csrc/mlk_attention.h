@@ -26,6 +26,21 @@ bool PrefillSupported(int32_t head_dim, const float* q, int64_t q_row_stride, co
 // multiple of 32), when set, also receives the output rows as StorePlanes
 // planes.
 constexpr int64_t kPrefillImageMinTokens = 128;
+// A prompt chunk whose token blocks are at most one workgroup per compute
+// unit, over a context of at least kPrefillSplitMinCtx positions, is split
+// over chunks of positions like decode tokens (LaunchDecodeTile): the number
+// of chunks of its n_pos positions (1: not split; at most TileChunk's for
+// max_ctx) and their length.  Llama-3-8B heads, whole ->
+// in chunks: 64 tokens at 4000 277 -> 42 us, 128 at 4000 197 -> 66, 389 at
+// 6000 303 -> 220; more blocks than units fill the chip by themselves (700 at
+// 2000: 154 whole, 233 in chunks).  Over short contexts the merge costs more
+// than the split gives (389 from position 0: 27 whole, 55 in chunks); over
+// 1000 positions it would gain (128 tokens 61 -> 39), but up to here a
+// call with a workspace keeps the sums of the prefill entry, which has none,
+// bit for bit.
+constexpr int64_t kPrefillSplitMinCtx = 2048;
+int64_t PrefillChunks(int64_t T, int32_t H, int32_t KV, int64_t n_pos, int64_t max_ctx,
+                      int* chunk);
 int64_t PrefillImageBytes(int32_t n_kv_heads, int32_t head_dim, int64_t n_pos);
 mlk_status LaunchPrefill(const float* q, int64_t q_row_stride, const float* kc, const float* vc,
                          int64_t slot, int32_t H, int32_t KV, int32_t head_dim, int32_t pos0,
@@ -38,13 +53,19 @@ mlk_status LaunchPrefill(const float* q, int64_t q_row_stride, const float* kc, 
 // one chunk it writes (acc, m, l) partials to ws_acc / ws_ml ([T, H, n_chunks,
 // hd] / [.., 2], n_chunks = ceil(max_ctx / chunk)) for AttnCombine; with one
 // it writes out.  Invalid positions raise err (their rows are zeroed by the
-// merge, or here with one chunk).  Arguments already validated.
+// merge, or here with one chunk).  images_at (consecutive positions,
+// head_dim 128): room for PrefillImageBytes(KV, head_dim, pos0 + T), used as
+// in LaunchPrefill.  Arguments already validated.
 int TileChunk(int64_t T, int32_t H, int32_t KV, int64_t max_ctx);
 mlk_status LaunchDecodeTile(const float* q, int64_t q_row_stride, const float* kc,
                             const float* vc, int64_t slot, int32_t H, int32_t KV,
                             int32_t head_dim, const int32_t* positions, int32_t pos0, int64_t T,
-                            int64_t max_ctx, float* out, float* ws_acc, float* ws_ml,
-                            int32_t* err, hipStream_t s);
+                            int64_t max_ctx, int chunk, float* out, float* ws_acc, float* ws_ml,
+                            int32_t* err, hipStream_t s, void* images_at = nullptr);
+
+// Workspace of a prompt chunk (positions == NULL, 16 or more tokens): chunk
+// partials and tile images, whichever its call uses.
+int64_t PromptAttentionBytes(int64_t T, int32_t H, int32_t KV, int32_t head_dim, int64_t max_ctx);
 
 // mlk_attention_decode_f32 with one more output: when the chunk merge runs
 // (more than one chunk of cache positions) and planes is not null, the merge

@@ -848,6 +848,21 @@ int64_t mlk_attention_workspace_bytes(int64_t n_tokens, int32_t n_heads, int32_t
 
 namespace mlk {
 
+namespace {
+// Chunk partials: (acc, m, l) per token, head and chunk.
+int64_t PartialBytes(int64_t T, int32_t H, int64_t n_chunks, int32_t head_dim) {
+    return T * H * n_chunks * (head_dim + 2) * static_cast<int64_t>(sizeof(float));
+}
+}  // namespace
+
+int64_t PromptAttentionBytes(int64_t T, int32_t H, int32_t KV, int32_t head_dim, int64_t max_ctx) {
+    int chunk = 0;
+    const int64_t nc = PrefillChunks(T, H, KV, max_ctx, max_ctx, &chunk);
+    int64_t b = nc > 1 ? (PartialBytes(T, H, nc, head_dim) + 255) / 256 * 256 : 0;
+    if (T >= kPrefillImageMinTokens) b += PrefillImageBytes(KV, head_dim, max_ctx);
+    return b;
+}
+
 mlk_status AttentionDecode(const float* q, int64_t q_row_stride, const float* k_cache,
                            const float* v_cache, int64_t n_layers, int64_t max_seq,
                            int32_t n_heads, int32_t n_kv_heads, int32_t head_dim, int64_t layer,
@@ -892,8 +907,19 @@ mlk_status AttentionDecode(const float* q, int64_t q_row_stride, const float* k_
         return Fail(MLK_ERR_INVALID, "%s: out must not alias q", fn);
     }
     const int64_t slot = static_cast<int64_t>(n_kv_heads) * head_dim;
-    if (positions == nullptr && n_tokens >= kPrefillMinTokens &&
-        PrefillSupported(head_dim, q, q_row_stride, out, k_cache, v_cache)) {
+    // a prompt chunk at consecutive positions, and whether it is split over
+    // chunks of positions (with room for their partial sums)
+    const bool prompt = positions == nullptr && n_tokens >= kPrefillMinTokens &&
+                        PrefillSupported(head_dim, q, q_row_stride, out, k_cache, v_cache);
+    int pchunk = 0;
+    const int64_t pnc = prompt ? PrefillChunks(n_tokens, n_heads, n_kv_heads, pos0 + n_tokens,
+                                               max_ctx, &pchunk)
+                               : 1;
+    const bool prompt_split =
+        pnc > 1 && workspace != nullptr && Aligned(workspace, 16) &&
+        static_cast<int64_t>(workspace_bytes) >=
+            PartialBytes(n_tokens, n_heads, pnc, head_dim);
+    if (prompt && !prompt_split) {
         // a prompt chunk at consecutive positions: the matrix-core prefill
         // kernel (a workspace of PrefillImageBytes holds the pre-split tiles)
         // (and a's planes, when asked, for a tiled wo)
@@ -908,11 +934,11 @@ mlk_status AttentionDecode(const float* q, int64_t q_row_stride, const float* k_
         // several decode tokens: 16 per workgroup share each K/V tile of a
         // chunk of positions (the prefill kernel's matrix-core tiles), then
         // AttnCombine merges the chunks
-        const int tchunk = TileChunk(n_tokens, n_heads, n_kv_heads, max_ctx);
-        const int64_t tnc = (max_ctx + tchunk - 1) / tchunk;
-        const int64_t need = tnc > 1 ? n_tokens * n_heads * tnc * (head_dim + 2) *
-                                           static_cast<int64_t>(sizeof(float))
-                                     : 0;
+        const int64_t n_ctx = prompt_split ? pos0 + n_tokens : max_ctx;
+        const int tchunk =
+            prompt_split ? pchunk : TileChunk(n_tokens, n_heads, n_kv_heads, max_ctx);
+        const int64_t tnc = (n_ctx + tchunk - 1) / tchunk;
+        const int64_t need = tnc > 1 ? PartialBytes(n_tokens, n_heads, tnc, head_dim) : 0;
         if (tnc > 1 && (workspace == nullptr || static_cast<int64_t>(workspace_bytes) < need)) {
             return Fail(MLK_ERR_INVALID, "%s: workspace of %lld bytes needed (got %zu)", fn,
                         static_cast<long long>(need), workspace_bytes);
@@ -921,15 +947,23 @@ mlk_status AttentionDecode(const float* q, int64_t q_row_stride, const float* k_
         float* ws_acc = tnc > 1 ? static_cast<float*>(workspace) : nullptr;
         float* ws_ml = tnc > 1 ? ws_acc + n_tokens * n_heads * tnc * head_dim : nullptr;
         const hipStream_t s = AsStream(stream);
+        // a prompt chunk's tile images, where they fit behind the partial sums
+        const int64_t images = (need + 255) / 256 * 256;
+        const int64_t image_bytes =
+            prompt_split ? PrefillImageBytes(n_kv_heads, head_dim, pos0 + n_tokens) : 0;
+        void* images_at = image_bytes > 0 && n_tokens >= kPrefillImageMinTokens &&
+                                  static_cast<int64_t>(workspace_bytes) >= images + image_bytes
+                              ? static_cast<char*>(workspace) + images
+                              : nullptr;
         st = LaunchDecodeTile(q, q_row_stride, k_cache + layer * max_seq * slot,
                               v_cache + layer * max_seq * slot, slot, n_heads, n_kv_heads,
-                              head_dim, positions, pos0, n_tokens, max_ctx, out, ws_acc, ws_ml,
-                              err, s);
+                              head_dim, positions, pos0, n_tokens, n_ctx, tchunk, out, ws_acc,
+                              ws_ml, err, s, images_at);
         if (st != MLK_OK || tnc == 1) return st;
         AttnParams p{};
         p.positions = positions;
         p.pos0 = pos0;
-        p.max_ctx = max_ctx;
+        p.max_ctx = n_ctx;
         p.H = n_heads;
         p.hd = head_dim;
         p.chunk = tchunk;

@@ -389,7 +389,7 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
     int64_t n_image_tiles, uint32_t* __restrict__ a_planes) {
 #pragma clang fp contract(off)
     static_assert(!kF16 || HD == 128, "fp16 products: head_dim 128");
-    static_assert(!kPre || (kF16 && !kChunked), "pre-split tiles: prompt chunks, fp16 products");
+    static_assert(!kPre || kF16, "pre-split tiles: fp16 products");
     static_assert(NBUF == 2 || (NBUF == 1 && kF16), "one tile buffer: fp16 products only");
     constexpr int LD = HD + 4;
     constexpr int NC = HD / 16;                          // 16-dim chunks
@@ -512,7 +512,7 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
             const MagScale mk(kk), mv(kv);
             k_factor = mk.f;
             v_exp = mv.fe;
-            if (!kChunked && max_pos - p0 < kPfTile - 1) tile.DropV(max_pos - p0);
+            if ((kPre || !kChunked) && max_pos - p0 < kPfTile - 1) tile.DropV(max_pos - p0);
             tile.Store(sm.k[buf], sm.v[buf], mk.s, mv.s);
         } else {
             tile.Store(sm.k[buf], sm.v[buf]);
@@ -787,15 +787,28 @@ int TileChunk(int64_t T, int32_t H, int32_t KV, int64_t max_ctx) {
     return static_cast<int>(chunk);
 }
 
+int64_t PrefillChunks(int64_t T, int32_t H, int32_t KV, int64_t n_pos, int64_t max_ctx,
+                      int* chunk) {
+    const int group = H / KV;
+    const int64_t base = (T + kPfTokens - 1) / kPfTokens * KV * ((group + kPfHeads - 1) / kPfHeads);
+    *chunk = 1 << 30;
+    if (base > ComputeUnits() || n_pos < kPrefillSplitMinCtx) return 1;
+    // by the positions there are, within the chunks of the workspace's sizing
+    const int max_chunk = TileChunk(T, H, KV, max_ctx);
+    const int64_t most = (max_ctx + max_chunk - 1) / max_chunk;
+    *chunk = TileChunk(T, H, KV, n_pos);
+    while ((n_pos + *chunk - 1) / *chunk > most) *chunk *= 2;
+    return (n_pos + *chunk - 1) / *chunk;
+}
+
 mlk_status LaunchDecodeTile(const float* q, int64_t q_row_stride, const float* kc,
                             const float* vc, int64_t slot, int32_t H, int32_t KV,
                             int32_t head_dim, const int32_t* positions, int32_t pos0, int64_t T,
-                            int64_t max_ctx, float* out, float* ws_acc, float* ws_ml,
-                            int32_t* err, hipStream_t s) {
+                            int64_t max_ctx, int chunk, float* out, float* ws_acc, float* ws_ml,
+                            int32_t* err, hipStream_t s, void* images_at) {
     const int group = H / KV;
     const int head_blocks = (group + kPfHeads - 1) / kPfHeads;
     const int64_t n_tb = (T + kPfTokens - 1) / kPfTokens;
-    const int chunk = TileChunk(T, H, KV, max_ctx);
     const int64_t nc = (max_ctx + chunk - 1) / chunk;
     const int64_t blocks = n_tb * KV * head_blocks * nc;
     if (blocks > 0x7FFFFFFF) return Fail(MLK_ERR_INVALID, "attention decode: launch too large");
@@ -806,6 +819,17 @@ mlk_status LaunchDecodeTile(const float* q, int64_t q_row_stride, const float* k
         hipLaunchKernelGGL((AttnPrefill<64, true, false>), grid, dim3(kPfThreads), 0, s, q,
                            q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
                            tc, nullptr, nullptr, 0, nullptr);
+    } else if (images_at != nullptr) {
+        // (consecutive positions) tiles from images, as LaunchPrefill
+        uint16_t* images = static_cast<uint16_t*>(images_at);
+        uint2* keys = nullptr;
+        int64_t n_tiles = 0;
+        const mlk_status st =
+            LaunchPieces(kc, vc, slot, KV, pos0 + T, images, &keys, &n_tiles, s);
+        if (st != MLK_OK) return st;
+        hipLaunchKernelGGL((AttnPrefill<128, true, true, 1, true>), grid, dim3(kPfThreads), 0, s, q,
+                           q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
+                           tc, images, keys, n_tiles, nullptr);
     } else if (blocks <= ComputeUnits()) {
         // two tile buffers (76 KB of LDS)
         hipLaunchKernelGGL((AttnPrefill<128, true, true>), grid, dim3(kPfThreads), 0, s, q,

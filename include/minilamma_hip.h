@@ -267,7 +267,12 @@ int64_t mlk_attention_workspace_bytes(int64_t n_tokens, int32_t n_heads, int32_t
  * from 128 tokens at head_dim 128, a 16-byte aligned workspace of at least
  * 12 * KV * head_dim * (pos0 + n_tokens rounded up to 32) bytes lets it split
  * K and V into fp16 pieces once (one extra launch) instead of in every
- * workgroup, with the same results; otherwise it uses no workspace.
+ * workgroup, with the same results.  From max_ctx 2048, when the chunk's
+ * blocks of 16 tokens are too few to fill the device, a 16-byte aligned
+ * workspace of mlk_attention_workspace_bytes() lets it split the positions
+ * over workgroups, partial sums merged as for decode tokens (the images then
+ * lie behind the partials, at the next 256 bytes).  Otherwise it uses no
+ * workspace.
  * Replaces CudaAttentionDevice (include/cuda_attention.h:12-13;
  * src/cuda_attention.cu:77-176, 2 launches, one cudaMalloc and a device
  * synchronize per call).
@@ -362,7 +367,9 @@ typedef struct {
  * tokens attending up to max_ctx positions; consecutive_positions != 0 when
  * the call passes positions == NULL (0 on bad input).  A prompt chunk of
  * 128 or more tokens at head_dim 128 includes the attention's pre-split
- * K/V (12 bytes per cached K and V element of a layer up to max_ctx). */
+ * K/V (up to 12 bytes per cached K and V element of a layer up to max_ctx);
+ * one of few tokens over 2048 or more positions, the attention's partial
+ * sums. */
 int64_t mlk_forward_layer_workspace_bytes(const mlk_layer_config* cfg, int64_t n_tokens,
                                           int64_t max_ctx, int32_t consecutive_positions);
 

@@ -651,6 +651,50 @@ def test_attention_tiles_of_far_apart_magnitudes(mlk, T, pos0):
         check(got[i], p - pos0, S - 1, "decode tiles")
 
 
+@pytest.mark.parametrize("H,KV,hd,T,pos0,spare", [
+    (8, 2, 128, 16, 2032, 0),     # 2048 positions: the first split context
+    (8, 2, 128, 17, 2030, 0),     # 2047: whole, the prefill entry's sums
+    (12, 2, 128, 127, 2500, 0),   # the last size without images; a partly idle head block
+    (8, 2, 128, 128, 2483, 9000), # images behind the partials; max_ctx far past the chunk
+    (8, 8, 64, 33, 2300, 40),     # head_dim 64, ragged blocks
+])
+def test_attention_prefill_split_over_positions(mlk, H, KV, hd, T, pos0, spare):
+    """A prompt chunk of few blocks over a long context, its positions split
+    over workgroups, in a workspace of exactly the documented size: against
+    float64 to the tiles' bound (merging two chunks rounds each sum three
+    times more at most, chunks of at least 256 positions, inside the n u of
+    the sums).  Slots past the chunk hold NaN.  Without a workspace the call
+    takes the prefill kernel, bit for bit."""
+    rng = np.random.default_rng(T + pos0)
+    n_pos = pos0 + T
+    S = n_pos + 40 + spare
+    kc, vc = random_cache(rng, 1, S, KV, hd)
+    kc[:, n_pos:] = np.nan
+    vc[:, n_pos:] = np.nan
+    cache = Cache(mlk, kc, vc)
+    q = rng.standard_normal((T, H, hd)).astype(np.float32)
+    max_ctx = n_pos + spare
+    whole = run_prefill(mlk, cache, q, 0, pos0)
+    d_q = mlk.DeviceBuffer.from_array(q)
+    part = (mlk.attention_workspace_bytes(T, H, KV, hd, max_ctx) + 255) // 256 * 256
+    got = {}
+    for name, size in (("none", 0), ("partials", part), ("images", part + image_bytes(KV, n_pos))):
+        out = mlk.DeviceBuffer.empty((T, H, hd))
+        ws = mlk.DeviceBuffer(max(size, 4), np.uint8) if size else None
+        mlk.attention_decode(d_q, cache.k, cache.v, 1, S, H, KV, hd, 0, T, out, max_ctx,
+                             pos0=pos0, workspace=ws, workspace_bytes=size)
+        got[name] = out.download()
+    np.testing.assert_array_equal(got["none"], whole)
+    if n_pos < 2048:
+        np.testing.assert_array_equal(got["images"], whole)
+    else:
+        assert (got["partials"] != whole).any(), "the positions were not split"
+    np.testing.assert_array_equal(got["images"], got["partials"])
+    ex, pav, dmax, n = prefill_exact(q, kc, vc, 0, pos0)
+    for name, o in got.items():
+        assert_prefill_close(o, ex, pav, dmax, n, name, pieces=hd == 128)
+
+
 def test_attention_prefill_rejects(mlk):
     kc = mlk.DeviceBuffer.empty((2, 64, 2, 128))
     vc = mlk.DeviceBuffer.empty((2, 64, 2, 128))
