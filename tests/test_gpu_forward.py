@@ -64,6 +64,29 @@ def test_tiny_model_prefill_then_decode_and_token_by_token(fwd):
         assert_forward_close(single.forward(tokens[t:t + 1], pos0=t), logits[t], f"token {t}")
 
 
+def test_forward_scratch_is_kept_across_calls(mlk, fwd):
+    """forward's buffers, kept by the model: calls of growing and shrinking
+    batches, with and without positions, on a stream and after a refused one
+    give what freshly allocated buffers give (hidden and logits), bit for bit;
+    scratch past the bound is not kept."""
+    model, tokens, positions, _ = tiny_model()
+    dm, ref = fwd.DeviceModel(model), fwd.DeviceModel(model)
+    stream = mlk.Stream()
+    for T, pos, all_rows, s in ((9, False, True, None), (3, True, True, None),
+                                (9, True, False, stream), (1, False, False, stream)):
+        p = np.arange(T, dtype=np.int32) if pos else None
+        want = ref.logits(ref.hidden(tokens[:T], positions=p), T if all_rows else 1).download()
+        got = dm.forward(list(tokens[:T]), positions=p, all_logits=all_rows, stream=s)
+        np.testing.assert_array_equal(got, want if all_rows else want[0])
+        kept = dm._scratch
+        assert kept is not None
+        with pytest.raises(mlk.MlkError):
+            dm.forward(tokens[:T], pos0=model["config"]["max_seq"])
+    dm._KEPT_SCRATCH = 0
+    dm.forward(tokens)
+    assert dm._scratch is None
+
+
 CASES = [  # config overrides, weight type, biases, tokens in the prefill batch
     (dict(dim=256, hidden_dim=512, n_heads=4, n_kv_heads=2, head_dim=64), "f32", True, 40),
     (dict(dim=256, hidden_dim=512, n_heads=4, n_kv_heads=2, head_dim=64), "q8_0", True, 40),
