@@ -126,7 +126,6 @@ class DeviceModel:
         self.k_cache.zero()
         self.v_cache.zero()
         self._ws = None
-        self._scratch = None  # forward's token, row and logits buffers (_take)
 
     def _up(self, a):
         a = np.ascontiguousarray(a)
@@ -220,11 +219,13 @@ class DeviceModel:
     # freeing the five, each free a wait for the device, took 65 of the 230 us
     # of a two-layer model of dim 32 on 9 tokens.
     _KEPT_SCRATCH = 64 << 20
+    _scratch = None
 
     def _take(self, n):
         """The kept scratch of at least n bytes, or a new one; a call takes it
-        out of the model, so calls on several threads never share one."""
-        buf, self._scratch = self._scratch, None
+        out of the model in one step (dict.pop), so calls on several threads
+        never share one."""
+        buf = self.__dict__.pop("_scratch", None)
         return buf if buf is not None and buf.nbytes >= n else DeviceBuffer(n, np.uint8)
 
     def forward(self, tokens, positions=None, pos0=0, all_logits=False, stream=None):
