@@ -51,10 +51,13 @@ int64_t Align256(int64_t bytes) { return (bytes + 255) / 256 * 256; }
 
 bool Contiguous(const int32_t* positions) { return positions == nullptr; }
 
-// Token counts whose linear layers run the skinny GEMM (8..32 rows): with
-// quantized weights the layer fuses them as the one-token path does, with
-// the epilogues in the split-K reduction.
-bool FusedRows(int64_t T) { return T >= 8 && T <= 32; }
+// Token counts whose quantized linear layers run the skinny GEMM (3..32
+// rows): the layer fuses them as the one-token path does, with the epilogues
+// in the split-K reduction.  Below 8 rows the GEMVs, which decode the weights
+// once per 4 rows, and their separate epilogue launches took 169 us for 4
+// tokens of the 8B layer (Q8_0 blocks) and 308 for 7, the skinny launches 124
+// and 137; for 2 tokens 109 against 123.
+bool FusedRows(int64_t T) { return T >= 3 && T <= 32; }
 
 // Token counts that take the planar weights when a layer has them (the
 // bf16 kernel, fused as FusedRows; one token keeps the block-layout GEMVs).
@@ -82,7 +85,7 @@ Plan MakePlan(const mlk_layer_config& c, int64_t T, int64_t max_ctx, bool contig
         if (b > p.lin_bytes) p.lin_bytes = b;
     }
     if (FusedRows(T)) {  // q/k/v, gate/up and down as fused skinny launches
-        const int64_t fused[3][2] = {{D, QD + 2 * KD}, {D, 2 * F}, {F, D}};  // (in, all outputs)
+        const int64_t fused[4][2] = {{D, QD + 2 * KD}, {D, 2 * F}, {F, D}, {QD, D}};  // (in, out)
         for (const auto& s : fused) {
             const int64_t b = SkinnyFusedWorkspaceBytes(MLK_Q8_0, T, s[0], s[1]);
             if (b > p.lin_bytes) p.lin_bytes = b;
@@ -90,7 +93,8 @@ Plan MakePlan(const mlk_layer_config& c, int64_t T, int64_t max_ctx, bool contig
     }
     for (const auto& g : {TileGroup{D, {QD, KD, KD}, 3}, TileGroup{QD, {D}, 1},
                           TileGroup{D, {F, F}, 2}, TileGroup{F, {D}, 1}}) {
-        if (!TileApplies(MLK_Q8_0, T, g.in)) continue;  // (planar copies are not used there)
+        // (planar copies, of up to 32 rows, are not used there)
+        if (T < 5 || !TileApplies(MLK_Q8_0, T, g.in)) continue;
         p.lin_bytes = std::max(p.lin_bytes, TileFusedPlan(T, g.in, g.rows, g.n).bytes);
     }
     if (PlanarRows(T)) {  // the same groups (and wo) on planar weights
@@ -287,7 +291,7 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
     // launch, gate and up with SwiGLU in the epilogue, and the down
     // projection adding into x (the same per-element arithmetic as the
     // separate kernels), over the planar copies where a group has them
-    // (contiguous loads), else over the blocks.  8..32 tokens: the same
+    // (contiguous loads), else over the blocks.  3..32 tokens: the same
     // groups as skinny GEMM launches, with the epilogues in their split-K
     // reductions.
     const hipStream_t hs = AsStream(stream);
@@ -308,29 +312,45 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
     const bool ffnp = Planar(T, D, {&w->w_gate, &w->w_up});
     const bool downp = Planar(T, F, {&w->w_down});
     const bool wop = Planar(T, QD, {&w->wo});
-    const bool mid = FusedRows(T);
-    const bool qkvm = qkvp || (mid && w->wq.type == w->wk.type && w->wq.type == w->wv.type &&
-                               w->wq.type != kLinearF32 && SkinnyFusedApplies(w->wq.type, T, D));
-    const bool ffnm = ffnp || (mid && w->w_gate.type == w->w_up.type &&
-                               w->w_gate.type != kLinearF32 &&
-                               SkinnyFusedApplies(w->w_gate.type, T, D));
-    const bool downm = downp || (mid && w->w_down.type != kLinearF32 &&
-                                 SkinnyFusedApplies(w->w_down.type, T, F));
-    // more than 32 tokens: the same groups on the tiled kernel, for any one
-    // weight type per group; a group's epilogue runs in the tiles where they
-    // fill the GPU without a K split, else in the split sums' reduction
-    const auto tiled = [&](int64_t in, std::initializer_list<const mlk_linear_weight*> ws) {
+    // where TileChosen says so: the same groups on the tiled kernel, for any
+    // one weight type per group; a group's epilogue runs in the tiles where
+    // they fill the GPU without a K split, else in the split sums' reduction
+    const auto tiled = [&](int64_t in, int64_t out,
+                           std::initializer_list<const mlk_linear_weight*> ws) {
         const int t = (*ws.begin())->type;
-        if (!TileApplies(t, T, in)) return false;
+        if (!TileChosen(t, T, in, out, true)) return false;
         for (const mlk_linear_weight* lw : ws) {
-            if (lw->type != t || !TileWeightAligned(t, lw->data)) return false;
+            if (lw->type != t || !TileWeightAligned(t, lw->data) ||
+                (T <= 32 && !Aligned(lw->data, 4))) {
+                return false;
+            }
         }
         return true;
     };
-    const bool qkv_t = !(qkv1 || qkvm) && tiled(D, {&w->wq, &w->wk, &w->wv});
-    const bool wo_t = !wop && !wo1p && tiled(QD, {&w->wo});
-    const bool ffn_t = !ffn1 && !ffnm && tiled(D, {&w->w_gate, &w->w_up});
-    const bool down_t = !down1 && !downm && tiled(F, {&w->w_down});
+    const bool qkv_t = !(qkv1 || qkvp) && tiled(D, QD + 2 * KD, {&w->wq, &w->wk, &w->wv});
+    const bool wo_t = !wop && !wo1p && tiled(QD, D, {&w->wo});
+    const bool ffn_t = !ffn1 && !ffnp && tiled(D, 2 * F, {&w->w_gate, &w->w_up});
+    const bool down_t = !down1 && !downp && tiled(F, D, {&w->w_down});
+    // else up to 32 tokens on the skinny kernel (quantized weights); below 8,
+    // blocks that are not 4-byte aligned keep the separate entries, and small
+    // groups below 5 (3 tokens through three layers of dim 512 169 -> 192 us;
+    // 5 tokens 245 -> 195)
+    const auto skinny = [&](int64_t in, int64_t out,
+                            std::initializer_list<const mlk_linear_weight*> ws) {
+        const int t = (*ws.begin())->type;
+        if (!FusedRows(T) || t == kLinearF32 || !SkinnyFusedApplies(t, T, in) ||
+            (T < 5 && in * out < kLayerGroupMin)) {
+            return false;
+        }
+        for (const mlk_linear_weight* lw : ws) {
+            if (lw->type != t || (T < 8 && !Aligned(lw->data, 4))) return false;
+        }
+        return true;
+    };
+    const bool qkvm = qkvp || (!qkv_t && skinny(D, QD + 2 * KD, {&w->wq, &w->wk, &w->wv}));
+    const bool ffnm = ffnp || (!ffn_t && skinny(D, 2 * F, {&w->w_gate, &w->w_up}));
+    const bool downm = downp || (!down_t && skinny(F, D, {&w->w_down}));
+    const bool wom = T < 8 && !wop && skinny(QD, D, {&w->wo});
     const int64_t qkv_rows[3] = {QD, KD, KD};
     const bool qkv_split = qkv_t && TileFusedPlan(T, D, qkv_rows, 3).splits > 1;
     // The fused q/k/v launches also rotate q and k (normal-layout pairs) and
@@ -463,6 +483,11 @@ mlk_status mlk_forward_layer_batch(const mlk_layer_config* cfg, const mlk_layer_
             sa.seg[0] = PlanarSeg(w->wo, proj, D);
             sa.n_seg = 1;
             MLK_TRY(LinearRowPlanar(w->wo.type, a, QD, sa, kStreamPlain, hs));
+        } else if (wom) {
+            StreamArgs sa{};
+            sa.seg[0] = Seg(w->wo, proj, D);
+            sa.n_seg = 1;
+            MLK_TRY(LinearSkinnyFused(w->wo.type, a, T, QD, sa, kStreamPlain, lin_ws, lin_b, hs));
         } else {
             MLK_TRY(Linear(w->wo, a, proj, T, QD, D, lin_ws, lin_b, stream));
         }

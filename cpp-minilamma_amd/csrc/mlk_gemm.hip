@@ -1334,7 +1334,7 @@ mlk_status ReduceSplitsFused(const float* partial, int splits, int64_t T, int64_
 }
 
 int64_t GemmWorkspaceBytes(int wt, int64_t T, int64_t K, int64_t O) {
-    if (TileApplies(wt, T, K)) return TileWorkspaceBytes(T, K, O);
+    if (TileChosen(wt, T, K, O, false)) return TileWorkspaceBytes(T, K, O);
     const SplitPlan p = SkinnyApplies(wt, T, K) ? PlanSkinny(wt, T, K) : PlanSplits(T, K, O);
     return p.splits > 1 ? static_cast<int64_t>(p.splits) * T * O * 4 : 0;
 }
@@ -1348,7 +1348,7 @@ int64_t GemmWorkspaceBytes(int wt, int64_t T, int64_t K, int64_t O) {
 mlk_status LaunchGemm(int wt, const float* x, const void* w, const float* bias, float* y,
                       int64_t T, int64_t K, int64_t O, int64_t row_bytes, void* workspace,
                       size_t workspace_bytes, hipStream_t s) {
-    if (TileApplies(wt, T, K)) {
+    if (TileChosen(wt, T, K, O, false)) {
         return LaunchTile(wt, x, w, bias, y, T, K, O, row_bytes, workspace, workspace_bytes, s);
     }
     const SplitPlan sk = PlanSkinny(wt, T, K);
@@ -1409,6 +1409,13 @@ mlk_status LaunchGemm(int wt, const float* x, const void* w, const float* bias, 
     mlk_status st = CheckLaunch("GemmMfma");
     if (st != MLK_OK || partial == nullptr) return st;
     return ReduceSplits(partial, plan.splits, bias, y, T, O, s);
+}
+
+bool SkinnyFewRows(int wt, int64_t T, int64_t K, int64_t O) {
+    if (wt == kWF32 || T < 3 || T > 7 || !SkinnyApplies(wt, T, K) || K * O < kFewRowsMin) {
+        return false;
+    }
+    return T >= 5 || O >= 3 * K;
 }
 
 bool SkinnyFusedApplies(int wt, int64_t T, int64_t K) {

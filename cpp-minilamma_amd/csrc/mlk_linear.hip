@@ -56,7 +56,8 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / kWave;
 constexpr int kMaxTok = 4;    // token rows per GEMV launch
-constexpr int kGemmMinRows = 8;  // from here on, the matrix-core GEMM (mlk_gemm.hip)
+constexpr int kGemmMinRows = 8;  // from here on, the matrix-core GEMM (mlk_gemm.hip); below,
+                                 // large matrices that FewRowsGemm names
 constexpr int kF32 = -1;      // QT value of F32 weights
 
 __device__ inline float WaveSumF(float v) {
@@ -1346,6 +1347,20 @@ __global__ __launch_bounds__(kMmTile* kMmTile) void MatmulKernel(const float* __
     if (row < M && col < N) c[row * N + col] = s;
 }
 
+// Calls below kGemmMinRows rows that the GEMM kernels serve faster, and
+// whether the workspace they need is there (else the GEMV, as before).
+bool FewRowsGemm(int wt, int64_t rows, int64_t K, int64_t O) {
+    return rows < kGemmMinRows &&
+           (wt == kF32 ? TileChosen(wt, rows, K, O, false) : SkinnyFewRows(wt, rows, K, O));
+}
+bool FewRowsGemmRoom(int wt, int64_t rows, int64_t K, int64_t O, const void* workspace,
+                     size_t workspace_bytes) {
+    if (!FewRowsGemm(wt, rows, K, O)) return false;
+    const int64_t need = GemmWorkspaceBytes(wt, rows, K, O);
+    return need == 0 || (workspace != nullptr && Aligned(workspace, 16) &&
+                         workspace_bytes >= static_cast<size_t>(need));
+}
+
 mlk_status CheckLinear(const char* fn, const float* x, const void* w, float* y, int64_t T,
                        int64_t K, int64_t O) {
     if (x == nullptr || w == nullptr || y == nullptr) {
@@ -1572,12 +1587,16 @@ using namespace mlk;
 extern "C" {
 
 int64_t mlk_linear_workspace_bytes(int64_t rows, int64_t in_features, int64_t out_features) {
-    if (rows < kGemmMinRows || rows <= 0 || in_features <= 0 || out_features <= 0) return 0;
+    if (rows < 3 || in_features <= 0 || out_features <= 0 ||
+        (rows < kGemmMinRows && in_features * out_features < kFewRowsMin)) {
+        return 0;
+    }
     // the plans differ by weight type (the skinny kernel's K chunk): the
     // larger serves every type
     int64_t most = 0;
     for (const int wt : {kF32, static_cast<int>(MLK_Q8_0), static_cast<int>(MLK_Q4_0),
                          static_cast<int>(MLK_Q4_1)}) {
+        if (rows < kGemmMinRows && !FewRowsGemm(wt, rows, in_features, out_features)) continue;
         const int64_t b = GemmWorkspaceBytes(wt, rows, in_features, out_features);
         if (b > most) most = b;
     }
@@ -1621,7 +1640,8 @@ mlk_status mlk_linear_quant(int32_t quant_type, const float* x, const void* w_bl
         }
         return CheckLaunch("GemvAnyKernel");
     }
-    if (rows >= kGemmMinRows) {
+    if (rows >= kGemmMinRows ||
+        FewRowsGemmRoom(quant_type, rows, K, O, workspace, workspace_bytes)) {
         return LaunchGemm(quant_type, x, w_blocks, bias, y, rows, K, O, row_bytes, workspace,
                           workspace_bytes, s);
     }
@@ -1654,7 +1674,7 @@ mlk_status mlk_linear_f32(const float* x, const float* w, const float* bias, flo
                            s, x, static_cast<const void*>(w), bias, y, K, O, K * 4, rows);
         return CheckLaunch("GemvAnyKernel");
     }
-    if (rows >= kGemmMinRows) {
+    if (rows >= kGemmMinRows || FewRowsGemmRoom(kF32, rows, K, O, workspace, workspace_bytes)) {
         return LaunchGemm(kF32, x, w, bias, y, rows, K, O, K * 4, workspace, workspace_bytes, s);
     }
     return Gemv<kF32>(x, reinterpret_cast<const uint8_t*>(w), bias, y, K, O, K * 4, K / 4, rows,

@@ -171,10 +171,34 @@ mlk_status ReduceSplits(const float* partial, int splits, const float* bias, flo
 mlk_status ReduceSplitsFused(const float* partial, int splits, int64_t T, int64_t cols,
                              const StreamArgs& a, int mode, hipStream_t s);
 
-// Many rows on the fp16 matrix cores (mlk_tile.hip): LaunchGemm's shapes
-// with more than 32 rows, K a multiple of 32 (planar: 256) and 256 or more.
-// Alignments and workspace as LaunchGemm.
+// Products on the fp16 matrix cores in tiles (mlk_tile.hip): K a multiple of
+// 32 (planar: 256) and 256 or more.  Alignments and workspace as LaunchGemm.
 bool TileApplies(int wt, int64_t T, int64_t K);
+// Where the tiles are the faster kernel, of a [cols, K] matrix or, fused, of
+// a layer's group of cols outputs: always above 32 rows, and below
+//   F32          from 8 rows (layer of 8 / 32 rows 319 -> 254 / 341 -> 267 us
+//                against the fp32 MFMA tiles), and from 5 where the weights
+//                are large (against the GEMV, which reads them once per 4
+//                rows: 7 rows of w_gate 105 -> 53 us, 4096 x 1024 9.6 -> 13.1);
+//   Q8_0, Q4_0   from 17 rows where the weights are large (32 rows, against
+//                the skinny kernel: 14336 x 4096 49 -> 35 us, 8192 x 8192 53
+//                -> 38, 4096 x 4096 17.6 -> 19.3, 4096 x 1024 11.9 -> 12.8;
+//                up to 16 rows that kernel has half the matrix work: 28 us
+//                for w_gate at 16 rows, 37 here).  A layer's groups already
+//                from 2^24: wo's reduction then is the norm's launch (layer,
+//                32 rows: Q8_0 209 -> 180 us).
+// Q4_1 up to 32 rows stays with the skinny kernel (w_gate 47 us, 50 here).
+constexpr int64_t kFewRowsMin = int64_t{1} << 25;     // weights of a large matrix
+constexpr int64_t kLayerGroupMin = int64_t{1} << 24;  // and of a layer's large group
+bool TileChosen(int wt, int64_t T, int64_t K, int64_t cols, bool fused);
+// A quantized matrix on the skinny kernel below 8 rows (with LaunchGemm's
+// workspace) instead of the GEMV, which decodes the weights once per 4 rows
+// and whose VALU is its bound from 3 on: 5..7 rows of large matrices (7 rows
+// of w_gate, Q8_0: 70 -> 27 us; 5 rows of w_down 41 -> 28), 3 and 4 rows
+// where the outputs are at least 3 times the inputs (few partial sums: 4
+// rows of w_gate 35 -> 27, 128256 outputs 288 -> 179; w_down, Q4_0, 24.5 ->
+// 29.6).  Small: 5 rows over 4096 x 1024 9.8 -> 11.0.
+bool SkinnyFewRows(int wt, int64_t T, int64_t K, int64_t O);
 int64_t TileWorkspaceBytes(int64_t T, int64_t K, int64_t O);
 mlk_status LaunchTile(int wt, const float* x, const void* w, const float* bias, float* y, int64_t T,
                       int64_t K, int64_t O, int64_t row_bytes, void* workspace,

@@ -1,7 +1,8 @@
 // mlk_tile.hip -- many-row linear layers on the fp16 matrix cores:
 // y[T, O] = x[T, K] W[O, K]^T (+ bias), W fp32, Q8_0 / Q4_0 / Q4_1 blocks or
-// planar Q8_0 / Q4_0, for more than 32 rows and K a multiple of 32, at least
-// 256 (other shapes: mlk_linear.hip, mlk_gemm.hip).  Semantics as there
+// planar Q8_0 / Q4_0, for more than 32 rows (F32 from 5, Q8_0 and Q4_0 blocks
+// from 17: TileChosen) and K a multiple of 32, at least 256 (other shapes:
+// mlk_linear.hip, mlk_gemm.hip).  Semantics as there
 // (LinearQ80 / Q40 / Q41, src/quant.cc:393-463; cublasSgemm,
 // src/cuda_matmul.cc:142-186): fp32 products and sums, in an order of this
 // kernel's choosing.
@@ -32,8 +33,8 @@
 // and its outputs are summed again in order in fp32 (SlowOutputs), so no
 // finite or infinite input is lost.  NaNs pass through the products.
 //
-// Work.  A workgroup owns BM token rows x BN outputs (64 x 128, 4 waves, or
-// 128 x 256, 8 waves), a wave a 16 MI x 16 NJ part of them, K in stages of 32
+// Work.  A workgroup owns BM token rows x BN outputs (32 x 64, 2 waves, 64 x
+// 128, 4 waves, or 128 x 256, 8 waves), a wave a 16 MI x 16 NJ part of them, K in stages of 32
 // through LDS; while stages are multiplied the next ones, already in
 // registers, are split, decoded and written to the other LDS buffers, and
 // the ones after them are requested from memory.  Few tiles: K is split over
@@ -719,6 +720,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
 //       splits (more while each keeps 16 stages) give 3/4 of a workgroup a
 //       CU; past that K is not split: T = 389 over 14336 outputs (224 tiles,
 //       Q8_0) took 150 us unsplit, 176 us in two splits of 1.75 rounds.
+//   32 x 64 up to 32 rows, split to 4 workgroups a CU (33 KB of LDS each),
+//       each split at least 8 stages.  16 rows of F32: w_gate 52 us (fp32
+//       MFMA 52), wo 19.9 (20.2); 32 rows of Q8_0 / Q4_0: w_gate 42 / 40 us
+//       (skinny kernel, fp32 MFMA, 48 / 47), 128256 outputs 263 / 216 (355 /
+//       366, whose 8 splits' partial sums alone are 131 MB).  On 64 x 128
+//       tiles the same take 46, 21.7, 40 / 39 and 265 / 228, Q8_0 wo 22 (19.3
+//       here).
 //   64 x 128 otherwise, split to 1.5 workgroups a CU, each split at least 8
 //       stages.  Q8_0: T = 64 over 4096 x 14336 39.6 us in 16 splits (512
 //       workgroups), 46 in 8; 128 rows over 4096 x 4096 31 us against 34-37
@@ -726,19 +734,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
 // Measured beside these: 128 x 128 tiles (4 waves) 7-14% slower than 128 x
 // 256 at every T from 200 to 4096.
 struct TilePlan {
-    bool wide = false;
+    int bm = 64;
     int splits = 1;
     int64_t per_split = 0, tiles_m = 0, tiles = 0;
-    int Bm() const { return wide ? 128 : 64; }
-    int Bn() const { return wide ? 256 : 128; }
+    int Bm() const { return bm; }
+    int Bn() const { return 2 * bm; }
 };
 
 // rows: outputs per segment; dual: gate and up in one tile
 TilePlan MakeTilePlan(int64_t T, int64_t K, const int64_t* rows, int n_seg, bool dual, bool split) {
     const int64_t cus = ComputeUnits(), stages = K / kBK;
     TilePlan p;
-    const auto count = [&](bool wide) {
-        p.wide = wide;
+    const auto count = [&](int bm) {
+        p.bm = bm;
         p.tiles_m = (T + p.Bm() - 1) / p.Bm();
         int64_t tn = 0;
         for (int i = 0; i < (dual ? 1 : n_seg); ++i) {
@@ -750,14 +758,15 @@ TilePlan MakeTilePlan(int64_t T, int64_t K, const int64_t* rows, int n_seg, bool
     int64_t sp = 1;
     bool wide = T > 64;
     if (wide) {
-        count(true);
+        count(128);
         while (p.tiles * sp * 4 < 3 * cus && stages / (2 * sp) >= 16 && sp < 32) sp *= 2;
         wide = p.tiles * sp * 4 >= 3 * cus;
     }
     if (!wide) {
-        count(false);
+        count(T <= 32 ? 32 : 64);
+        const int64_t half_wgs = T <= 32 ? 8 : 3;  // per CU
         sp = 1;
-        while (p.tiles * sp * 2 < 3 * cus && stages / (2 * sp) >= 8 && sp < 32) sp *= 2;
+        while (p.tiles * sp * 2 < half_wgs * cus && stages / (2 * sp) >= 8 && sp < 32) sp *= 2;
     }
     if (!split) sp = 1;
     p.per_split = (stages + sp - 1) / sp;
@@ -771,11 +780,17 @@ void LaunchEpi(const TilePlan& p, hipStream_t s, const TileArgs& a) {
     const dim3 grid(static_cast<unsigned>(p.tiles * p.splits));
     constexpr int kPair = kCodes<WT> ? 2 : 1;
     const bool pair = kCodes<WT> && a.K % 64 == 0;
-    if (p.wide) {
+    if (p.bm == 128) {
         if (pair) {
             hipLaunchKernelGGL((GemmTile<WT, 4, 4, 2, 4, EPI, kPair>), grid, dim3(512), 0, s, a);
         } else {
             hipLaunchKernelGGL((GemmTile<WT, 4, 4, 2, 4, EPI, 1>), grid, dim3(512), 0, s, a);
+        }
+    } else if (p.bm == 32) {
+        if (pair) {
+            hipLaunchKernelGGL((GemmTile<WT, 2, 2, 1, 2, EPI, kPair>), grid, dim3(128), 0, s, a);
+        } else {
+            hipLaunchKernelGGL((GemmTile<WT, 2, 2, 1, 2, EPI, 1>), grid, dim3(128), 0, s, a);
         }
     } else if (pair) {
         hipLaunchKernelGGL((GemmTile<WT, 2, 4, 2, 2, EPI, kPair>), grid, dim3(256), 0, s, a);
@@ -834,8 +849,16 @@ bool WorkspaceOk(const void* workspace, size_t bytes, int64_t need) {
 
 bool TileApplies(int wt, int64_t T, int64_t K) {
     // the 32-bit row offsets of a tile hold 256 rows of 2^22 fp32 inputs
-    return T > 32 && K >= 256 && K <= (int64_t{1} << 22) &&
+    return T > 0 && K >= 256 && K <= (int64_t{1} << 22) &&
            K % (wt == kWPlanarQ8 || wt == kWPlanarQ4 ? 256 : 32) == 0;
+}
+
+bool TileChosen(int wt, int64_t T, int64_t K, int64_t cols, bool fused) {
+    if (!TileApplies(wt, T, K)) return false;
+    if (T > 32) return true;
+    const int64_t n = K * cols;
+    if (wt == kWF32) return T >= 8 || (T >= 5 && n >= kFewRowsMin);
+    return (wt == MLK_Q8_0 || wt == MLK_Q4_0) && T > 16 && n >= (fused ? kLayerGroupMin : kFewRowsMin);
 }
 
 bool TileWeightAligned(int wt, const void* w) {

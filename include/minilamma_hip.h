@@ -171,8 +171,8 @@ mlk_status mlk_linear_f32(const float* x, const float* w, const float* bias, flo
 
 /* Device bytes of the optional workspace of mlk_linear_quant / mlk_linear_f32
  * for this shape on the current device (0: the call uses none).  Calls of
- * 8 rows or more run on the matrix cores in output tiles; when those tiles
- * are too few to fill the compute units, a workspace of this size
+ * 8 rows or more, and of 3 or more over large matrices, run on the matrix
+ * cores in output tiles; when those tiles are too few to fill the compute units, a workspace of this size
  * (16-byte aligned, not aliasing x, W or y) lets the call split K over
  * workgroups and add the partial sums in a fixed order.  Without it (NULL or
  * smaller) the call is still correct, only slower.  No counterpart in the

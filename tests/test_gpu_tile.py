@@ -1,5 +1,7 @@
-"""The many-row linear kernel on fp16 pieces (csrc/mlk_tile.hip): more than 32
-rows, in_features a multiple of 32 and at least 256.
+"""The linear kernel on fp16 pieces (csrc/mlk_tile.hip), in_features a multiple
+of 32 and at least 256: more than 32 rows; F32 from 5 rows and Q8_0 / Q4_0
+blocks from 17 where the weights are large; and the skinny kernel's calls
+below 8 rows.
 
 Bar: every output within gamma_K * sum_k |x_k w_k| of the float64 product
 with the dequantized weights (conftest.assert_dot_close).  A product here is
@@ -122,6 +124,64 @@ def test_tile_layer_matches_oracle(orc, mlk, wt, gaps):
                head_dim=64, max_seq=256, rope_type=0, theta=10000.0, eps=1e-5)
     model = O.forward_model(cfg, seed=5, weight_type=wt, biases=True)
     T = 70
+    tokens = (np.arange(T, dtype=np.int32) * 11 + 3) % 200
+    pos = np.cumsum(np.arange(T) % 4 + 1 if gaps else np.ones(T)).astype(np.int32) - 1
+    want, _ = orc.forward_tokens(model, tokens, pos)
+    dm = fwd.DeviceModel(model)
+    x = dm.hidden(tokens, positions=pos if gaps else None)
+    got = dm.logits(x, T).download().astype(np.float64)
+    assert (np.abs(got - want) <= 1e-5 + 1e-4 * np.abs(want)).all()
+
+
+# (kind, out, in, rows): both sides of each rule of up to 32 rows (2^25
+# weights and 5 / 17 rows; outputs 3 times the inputs for 3 and 4), remainders
+# of the 32 x 64 tiles and of the skinny kernel's 64 outputs
+FEW = [("f32", 63, 288, 8), ("f32", 65, 4128, 17), ("f32", 4097, 512, 32),
+       ("f32", 32769, 1024, 5), ("f32", 32767, 1024, 5), ("f32", 32768, 1024, 7),
+       ("q8_0", 32769, 1024, 17), ("q4_0", 8193, 4128, 31), ("q8_0", 32768, 1024, 32),
+       ("q4_0", 32768, 1024, 16), ("q8_0", 8192, 4096, 5), ("q4_0", 8193, 4096, 7),
+       ("q4_1", 8193, 4096, 6), ("q4_1", 12289, 2816, 3), ("q8_0", 12289, 2816, 4),
+       ("q4_0", 12288, 2816, 3), ("q8_0", 8192, 4096, 4), ("q8_0", 8191, 4096, 7)]
+
+
+@pytest.mark.parametrize("kind,out,K,T", FEW)
+def test_few_rows(mlk, orc, kind, out, K, T):
+    """Up to 32 rows, with the workspace and without one (unsplit, or below 8
+    rows the GEMV), against the same bar; with it also a zero row, a row out
+    of the pieces' range, infinite and NaN values.  (The GEMV's Q4_1 sums are
+    d sum(code x) + m sum(x), whose error follows |d code x| + |m x|, not
+    |x w|: no outlier there.)"""
+    rng = np.random.default_rng(out + K + T)
+    w, x, bias = normal(rng, (out, K), 0.02), normal(rng, (T, K)), normal(rng, (out,), 0.1)
+    for workspace in (None, "auto"):
+        if workspace == "auto":
+            x[1] = 0
+            x[2, 100] = 5e5
+        got, wd = run(mlk, orc, kind, x, w, bias, workspace)
+        ex, s = dot_exact(x, wd, bias)
+        assert_dot_close(got, ex, s, K + 1, f"{kind} {(out, K, T)} workspace={workspace}")
+    x[0, 3], x[2, 200] = np.inf, np.nan
+    got, wd = run(mlk, orc, kind, x, w, bias)
+    with np.errstate(invalid="ignore"):
+        want = x.astype(np.float64) @ wd.astype(np.float64).T
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(got[0], want[0].astype(np.float32))
+
+
+@pytest.mark.parametrize("wt,T", [("q8_0", 3), ("q4_0", 7), ("q4_1", 5), ("f32", 5), ("f32", 8),
+                                  ("q8_0", 17), ("q4_0", 32)])
+@pytest.mark.parametrize("gaps", [False, True])
+def test_few_row_layer_matches_oracle(orc, mlk, wt, T, gaps):
+    """A layer's fused launches on up to 32 tokens: skinny from 3 (wo too
+    below 8), tiles for F32 and, where a group has 2^24 weights (gate and up
+    here), for Q8_0 / Q4_0 from 17."""
+    import importlib
+    fwd = importlib.import_module(mlk.__name__ + ".forward")
+    big = T > 16
+    cfg = dict(vocab=200, dim=1024 if big else 512, hidden_dim=8192 if big else 1024, layers=2,
+               n_heads=8, n_kv_heads=2, head_dim=64, max_seq=256, rope_type=0, theta=10000.0,
+               eps=1e-5)
+    model = O.forward_model(cfg, seed=T, weight_type=wt, biases=True)
     tokens = (np.arange(T, dtype=np.int32) * 11 + 3) % 200
     pos = np.cumsum(np.arange(T) % 4 + 1 if gaps else np.ones(T)).astype(np.int32) - 1
     want, _ = orc.forward_tokens(model, tokens, pos)
