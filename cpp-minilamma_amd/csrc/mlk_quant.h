@@ -176,17 +176,19 @@ mlk_status ReduceSplitsFused(const float* partial, int splits, int64_t T, int64_
 bool TileApplies(int wt, int64_t T, int64_t K);
 // Where the tiles are the faster kernel, of a [cols, K] matrix or, fused, of
 // a layer's group of cols outputs: always above 32 rows, and below
-//   F32          from 8 rows (layer of 8 / 32 rows 319 -> 254 / 341 -> 267 us
-//                against the fp32 MFMA tiles), and from 5 where the weights
-//                are large (against the GEMV, which reads them once per 4
-//                rows: 7 rows of w_gate 105 -> 53 us, 4096 x 1024 9.6 -> 13.1);
+//   F32          from 8 rows (layer of 8 / 32 rows 304 -> 253 / 320 -> 274 us
+//                against the fp32 MFMA tiles; alone, where a layer's values
+//                are to be the same, 16 rows of w_gate 51.2 -> 50.6, of wo
+//                19.6 -> 21.4), and from 5 where the weights are large
+//                (against the GEMV, which reads them once per 4 rows: 7 rows
+//                of w_gate 104 -> 51 us, 4096 x 1024 9.6 -> 13.1);
 //   Q8_0, Q4_0   from 17 rows where the weights are large (32 rows, against
-//                the skinny kernel: 14336 x 4096 49 -> 35 us, 8192 x 8192 53
-//                -> 38, 4096 x 4096 17.6 -> 19.3, 4096 x 1024 11.9 -> 12.8;
-//                up to 16 rows that kernel has half the matrix work: 28 us
-//                for w_gate at 16 rows, 37 here).  A layer's groups already
-//                from 2^24: wo's reduction then is the norm's launch (layer,
-//                32 rows: Q8_0 209 -> 180 us).
+//                the skinny kernel: w_gate 49.5 -> 41.7 us, 8192 x 8192 51 ->
+//                34, 4096 x 4096 17.6 -> 19.3, 4096 x 1024 11.9 -> 12.8; up to
+//                16 rows that kernel has half the matrix work: 28 us for
+//                w_gate at 16 rows, 37 here).  A layer's groups already from
+//                2^24: wo's reduction then is the norm's launch (layer, 32
+//                rows: Q8_0 196 -> 165 us).
 // Q4_1 up to 32 rows stays with the skinny kernel (w_gate 47 us, 50 here).
 constexpr int64_t kFewRowsMin = int64_t{1} << 25;     // weights of a large matrix
 constexpr int64_t kLayerGroupMin = int64_t{1} << 24;  // and of a layer's large group

@@ -1,49 +1,69 @@
 // mlk_tile.hip -- many-row linear layers on the fp16 matrix cores:
 // y[T, O] = x[T, K] W[O, K]^T (+ bias), W fp32, Q8_0 / Q4_0 / Q4_1 blocks or
 // planar Q8_0 / Q4_0, for more than 32 rows (F32 from 5, Q8_0 and Q4_0 blocks
-// from 17: TileChosen) and K a multiple of 32, at least 256 (other shapes:
-// mlk_linear.hip, mlk_gemm.hip).  Semantics as there
+// from 17 where the weights are large: TileChosen) and K a multiple of 32, at
+// least 256 (other shapes: mlk_linear.hip, mlk_gemm.hip).  Semantics as there
 // (LinearQ80 / Q40 / Q41, src/quant.cc:393-463; cublasSgemm,
 // src/cuda_matmul.cc:142-186): fp32 products and sums, in an order of this
 // kernel's choosing.
 //
 // Products.  Each row of x (and of fp32 or Q4_1 weights, decoded to the
-// reference's fp32 values) is scaled by a power of two and split into two
-// fp16 pieces, the value rounded to fp16 and the rest rounded to fp16:
-// together the value to within one unit of its fp32 last place.
-//   codes (Q8_0, Q4_0)    a code is a small integer, exact in fp16, so a
-//       block's sum S = sum code (x0 + x1) is two v_mfma_f32_16x16x32_f16,
-//       then acc += d S + d' S' for a pair of blocks, in fp32 (one rounding
-//       of acc for two blocks: with one per block the sums were 2.2e-7 off
-//       at K = 4096 instead of 1.7e-7, and the kernel 5% faster).
-//   values (F32, Q4_1)    x1 w0 + x0 w1 + x0 w0, three MFMAs straight into
-//       the accumulators; x1 w1, below 2^-22 of the product, is left out.
+// reference's fp32 values) is scaled by a power of two s and split into two
+// fp16 pieces: x s = x0 + 2^-11 x1, x0 the value rounded to fp16, x1 the rest
+// times 2^11 rounded to fp16.  Where |x s| >= 2^-14 the pieces hold it to
+// 2^-23 of itself, below to 2^-36.
+//   codes (Q8_0, Q4_0)    a code is a small integer, exact in fp16 also
+//       times 2^-11, so a block's sum S = sum (code x0 + (2^-11 code) x1) is
+//       two v_mfma_f32_16x16x32_f16, then acc += d S + d' S' for a pair of
+//       blocks, in fp32 (one rounding of acc for two blocks: with one per
+//       block the sums were 2.2e-7 off at K = 4096 instead of 1.7e-7, and the
+//       kernel 5% faster).
+//   values (F32, Q4_1)    S = x1 w0 + x0 w1, acc += x0 w0 (three MFMAs), then
+//       acc += 2^-11 S; x1 w1 is left out.  (S kept over all stages instead:
+//       within 1% at 8 rows of F32, Q4_1 437 -> 466 us at 800 rows.)
 // Three bf16 pieces per x (exact products) and the fp32 MFMA, which these
 // replace, took 3 and, at an eighth of the rate, 8 times the matrix work.
 // Errors against float64 (relative 2-norm, normal x and weights, K = 4096
-// unsplit): Q8_0 1.7e-7 (three pieces: 2.1e-7), F32 7.1e-7 and Q4_1 6.8e-7
-// (fp32 MFMA: 1.1e-6).  Time at 4096 rows, K = 4096, 14336 outputs: Q8_0 1366
-// -> 1170 us, F32 3649 -> 1460, Q4_1 3807 -> 1450; at 64 rows Q8_0 91 -> 41.
+// unsplit): Q8_0 1.7e-7 (three pieces: 2.1e-7), F32 and Q4_1 4.6e-7 (fp32
+// MFMA: 1.15e-6).  Time at 4096 rows, K = 4096, 14336 outputs: Q8_0 1363 ->
+// 1217 us, F32 3659 -> 1678, Q4_1 3827 -> 1551; at 64 rows Q8_0 91 -> 43.
 //
-// Scales.  A row's power of two puts the mean magnitude of its first 64
-// inputs in [2, 4): fp16 then holds values up to 16000 times that mean, and
-// the second piece's subnormals reach 2^-25.  Every thread keeps the largest
-// magnitude of the rows it loads; a row whose largest scaled value leaves
-// [2^-3, 65504), infinities among them, is marked at the end of the K loop
-// and its outputs are summed again in order in fp32 (SlowOutputs), so no
-// finite or infinite input is lost.  NaNs pass through the products.
+// Scales and range.  s puts the largest of a row's first 64 inputs of the K
+// split (where those are zero, the first that are not of 64 at 7 places
+// further on) at [2^7, 2^8), weights' at [2^10, 2^11).  Every thread keeps the
+// largest and the smallest nonzero magnitude of the rows it loads, in fp32 (of
+// Q4_1 blocks bounds of both from d and m).  After the K loop a row is marked
+// unless every value is below 65504 / s (infinities are not) and every nonzero
+// one at least 2^-11 / (K s), for values 2^-10 / (K s); and for values also a
+// row of x whose smallest scaled magnitude times the tile's smallest is below
+// 2^-25 / K.  A product of an unmarked output is then within
+//   codes   (4 + K / 2) u |x w|, the K only for x at that lower bound (the
+//           pieces' 2^-36 against it; u = 2^-24)
+//   values  (8 + K / 4 + K / 4 + K / 2) u |x w|, the terms in K for x and w at
+//           the lower bounds and x1 w1 (up to 2^-50) at the bound of the pair
+// of its exact value, whatever the row's other values are and whichever of
+// them meet weights of zero.  Marked outputs are summed again as fp32 products
+// (MarkedRow, MarkedOutputs).  A row's values do not depend on the tile's other
+// rows, but for the order of a marked row's sums (one for up to 8 marked rows,
+// one for more).  Rows are marked that reach about 2^8 above or 2^(18 + log2 K)
+// below their first inputs; of normal rows about one in 10^5, of SwiGLU's
+// outputs one in 10^4.  Time (Q8_0, 4096 rows, K = 4096, 14336 outputs): one
+// marked row in every tile 1217 -> 1540 us, all rows marked 7160; first inputs
+// zero: no difference.  NaNs pass through the products.  Keeping both
+// magnitudes takes about 4% of the call, scaling the second pieces 3%.
 //
 // Work.  A workgroup owns BM token rows x BN outputs (32 x 64, 2 waves, 64 x
-// 128, 4 waves, or 128 x 256, 8 waves), a wave a 16 MI x 16 NJ part of them, K in stages of 32
-// through LDS; while stages are multiplied the next ones, already in
+// 128, 4 waves, or 128 x 256, 8 waves), a wave a 16 MI x 16 NJ part of them,
+// K in stages of 32 through LDS; while stages are multiplied the next ones, already in
 // registers, are split, decoded and written to the other LDS buffers, and
 // the ones after them are requested from memory.  Few tiles: K is split over
 // workgroups, partial sums reduced in split order (mlk_gemm.hip).
 //
-// Bound: a stage of a 128 x 256 tile (T = 4096, Q8_0) takes about 2800
-// cycles where its MFMAs take 1024 a SIMD; without the loads from memory 2080,
-// without loads, splits, decodes and LDS writes 1850, the scale FMAs 190 of
-// it (timing-only copies).  Not the order of instructions, deeper requests (3
+// Bound: a stage of a 128 x 256 tile (T = 4096, Q8_0) takes about 2900
+// cycles where its MFMAs take 1024 a SIMD; before the range was kept and the
+// second pieces scaled 2800, then without the loads from memory 2080, without
+// loads, splits, decodes and LDS writes 1850, the scale FMAs 190 of it
+// (timing-only copies).  Not the order of instructions, deeper requests (3
 // and 4 stages ahead), coalesced weight pieces through LDS, or the two halves
 // of the waves half a stage apart: each the same or slower.
 #include "mlk_quant.h"
@@ -56,6 +76,7 @@ namespace {
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef uint16_t us2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
@@ -69,29 +90,31 @@ constexpr bool kCodes = WT == MLK_Q8_0 || WT == MLK_Q4_0 || WT == kWPlanarQ8 || 
 template <int WT>
 constexpr bool kPlanar = WT == kWPlanarQ8 || WT == kWPlanarQ4;
 
+constexpr float kLowUp = 2048.0f;  // second pieces are kept times 2^11
+
 __device__ inline uint32_t AsU32(h2 v) { return __builtin_bit_cast(uint32_t, v); }
 
 // ------------------------------------------------------------ fp16 pieces
-// v * s = p0 + p1 + (at most one unit in the last place of fp32), p0 and p1
-// fp16; 8 values, two a dword.
+// v s = p0 + 2^-11 p1 (+ at most 2^-23 of v s, or 2^-36 where that is more),
+// p0 and p1 fp16; 8 values, two a dword.  (The asm hides where p0 came from,
+// which would otherwise be rounded twice: Q8_0 at 4096 rows 1203 -> 1183 us.)
 __device__ inline void Split8(const float4 (&v)[2], float s, u32x4* p0, u32x4* p1) {
     const float f[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
+    const float s2 = s * kLowUp;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const float a = f[2 * i], b = f[2 * i + 1];
+        const float a = f[2 * i] * s2, b = f[2 * i + 1] * s2;
         h2 hi, lo;
-        hi.x = static_cast<_Float16>(a * s);
-        hi.y = static_cast<_Float16>(b * s);
-        lo.x = static_cast<_Float16>(fmaf(a, s, -static_cast<float>(hi.x)));
-        lo.y = static_cast<_Float16>(fmaf(b, s, -static_cast<float>(hi.y)));
-        (*p0)[i] = AsU32(hi);
+        hi.x = static_cast<_Float16>(a * (1.0f / kLowUp));
+        hi.y = static_cast<_Float16>(b * (1.0f / kLowUp));
+        uint32_t u = AsU32(hi);
+        asm("" : "+v"(u));
+        hi = __builtin_bit_cast(h2, u);
+        lo.x = static_cast<_Float16>(fmaf(static_cast<float>(hi.x), -kLowUp, a));
+        lo.y = static_cast<_Float16>(fmaf(static_cast<float>(hi.y), -kLowUp, b));
+        (*p0)[i] = u;
         (*p1)[i] = AsU32(lo);
     }
-}
-
-__device__ inline float AbsSum8(const float4 (&v)[2]) {
-    return ((fabsf(v[0].x) + fabsf(v[0].y)) + (fabsf(v[0].z) + fabsf(v[0].w))) +
-           ((fabsf(v[1].x) + fabsf(v[1].y)) + (fabsf(v[1].z) + fabsf(v[1].w)));
 }
 
 __device__ inline float AbsMax8(const float4 (&v)[2], float m) {
@@ -103,22 +126,39 @@ __device__ inline float AbsMax8(const float4 (&v)[2], float m) {
     return m;
 }
 
-// The power of two that brings `mean` into [2, 4) and its inverse (within
-// 2^-61 .. 2^61; 1 for zero, subnormal, infinite and NaN means).
+// Smallest magnitude but zero, as a key that orders like it (infinities and
+// NaNs above every finite value, zero above all).
+constexpr uint32_t kNoKey = 0xFFFFFFFFu;
+__device__ inline uint32_t LeastKey(float v) { return (__float_as_uint(v) << 1) - 1u; }
+__device__ inline uint32_t LeastKey8(const float4 (&v)[2], uint32_t m) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        m = min(min(m, LeastKey(v[i].x)), LeastKey(v[i].y));
+        m = min(min(m, LeastKey(v[i].z)), LeastKey(v[i].w));
+    }
+    return m;
+}
+__device__ inline float KeyValue(uint32_t k) {
+    return k == kNoKey ? INFINITY : __uint_as_float((k + 1u) >> 1);
+}
+
+// The power of two that brings `first`, the largest magnitude of a row's
+// first inputs, into [2^at, 2^(at + 1)) and its inverse (2^at for zero,
+// subnormal, infinite and NaN values; within 2^(at - 61) .. 2^(at + 61)).  x
+// takes at = 7: room for activations of 250 times that magnitude; weights 10.
 struct PieceScale {
     float s = 1.0f, inv = 1.0f;
     __device__ PieceScale() {}
-    __device__ explicit PieceScale(float mean) {
-        int e = static_cast<int>((__float_as_uint(mean) >> 23) & 255u);
-        e = e == 0 || e == 255 ? 128 : (e < 66 ? 66 : (e > 188 ? 188 : e));
-        s = __uint_as_float(static_cast<uint32_t>(255 - e) << 23);
-        inv = __uint_as_float(static_cast<uint32_t>(e - 1) << 23);
+    __device__ PieceScale(float first, int at) {
+        int e = static_cast<int>((__float_as_uint(first) >> 23) & 255u);
+        e = e == 0 || e == 255 ? 127 : (e < 66 ? 66 : (e > 188 ? 188 : e));
+        s = __uint_as_float(static_cast<uint32_t>(254 + at - e) << 23);
+        inv = __uint_as_float(static_cast<uint32_t>(e - at) << 23);
     }
-    // inv, or 0 when the row's largest magnitude leaves the pieces' range
-    // (all zero stays in it)
-    __device__ float Checked(float most) const {
-        const float m = most * s;
-        return m == 0.0f || (m >= 0.125f && m < 65504.0f) ? inv : 0.0f;
+    // whether a row's values lie in the pieces' range: its largest magnitude
+    // and its smallest but zero
+    __device__ bool Fits(float most, float least, float low_min) const {
+        return most == 0.0f || (most * s < 65504.0f && least * s >= low_min);
     }
 };
 
@@ -216,43 +256,90 @@ __device__ inline void Values16(const RawW<MLK_Q4_1>& r, int h, float4 (&v)[2][2
     }
 }
 
-// One weight of row o (SlowOutputs).
+// A Q4_1 block's range from its scale d and minimum m: no value is above
+// |m| + 15 |d|, and as a multiple of the spacing of both no value but zero is
+// below the smaller spacing (2^(e - 25) at exponent field e).
+__device__ inline float BlockMost(const RawW<MLK_Q4_1>& r) {
+    return fmaf(15.0f, fabsf(HalfHw(r.d & 0xFFFFu)), fabsf(HalfHw(r.d >> 16)));
+}
+// both magnitudes less one: zero above all
+__device__ inline us2 BlockKeys(const RawW<MLK_Q4_1>& r) {
+    return __builtin_bit_cast(us2, r.d & 0x7FFF7FFFu) - us2{1, 1};
+}
+__device__ inline float KeySpacing(us2 k) {
+    const uint32_t m = k.x < k.y ? k.x : k.y;
+    if (m == 0xFFFFu) return INFINITY;
+    const uint32_t e = (m + 1u) >> 10;
+    return __uint_as_float((102u + (e > 0 ? e : 1)) << 23);
+}
+
+// 8 weights of row o in block kb: inputs e .. e + 3 and 16 + e .. 16 + e + 3
+// of its 32 (e = 0, 4, 8 or 12), as loaded and as the reference's fp32 values
+// (codes: exact).
 template <int WT>
-__device__ inline float Weight(const uint8_t* w, int64_t O, int64_t K, int64_t row_bytes,
-                               int64_t o, int64_t k) {
-    const int64_t kb = k / 32;
-    const int e = static_cast<int>(k % 32);
-    if constexpr (WT == kWF32) {
-        return reinterpret_cast<const float*>(w + o * row_bytes)[k];
-    } else if constexpr (WT == kWPlanarQ8 || WT == kWPlanarQ4) {
-        const int64_t rt = o / 16, r = o % 16;
-        const int64_t tile = (WT == kWPlanarQ8 ? 16 : 8) * K;
-        const int lane = 16 * (e / 8) + static_cast<int>(r), e8 = e % 8;
-        const uint8_t* s = w + (O + 15) / 16 * tile + ((rt * (K / 256) + kb / 8) * 16 + r) * 16;
-        const float d = HalfHw(reinterpret_cast<const uint16_t*>(s)[kb % 8]);
-        if constexpr (WT == kWPlanarQ8) {
-            const uint8_t* c = w + rt * tile + ((kb / 2) * 64 + lane) * 16 + (kb & 1) * 8;
-            return d * static_cast<float>(static_cast<int8_t>(c[e8]));
+struct Raw8 {
+    uint32_t d, u[2];  // scale (Q4_1: and minimum), 4 codes each
+    __device__ void Load(const uint8_t* w, int64_t O, int64_t K, int64_t row_bytes, int64_t o,
+                         int64_t kb, int e) {
+        typedef uint32_t u32_a2 __attribute__((aligned(2)));
+        if constexpr (kPlanar<WT>) {
+            const int64_t rt = o / 16, r = o % 16;
+            const int64_t tile = (WT == kWPlanarQ8 ? 16 : 8) * K;
+            const uint8_t* s = w + (O + 15) / 16 * tile;
+            d = *reinterpret_cast<const uint16_t*>(
+                s + ((rt * (K / 256) + kb / 8) * 16 + r) * 16 + kb % 8 * 2);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {  // 8 inputs from 16 c + e / 8 * 8 on
+                const int64_t at = 16 * (2 * c + e / 8) + r;
+                const uint8_t* q =
+                    WT == kWPlanarQ8 ? w + rt * tile + (kb / 2 * 64 + at) * 16 + kb % 2 * 8 + e % 8
+                                     : w + rt * tile + (kb / 4 * 64 + at) * 16 + kb % 4 * 4;
+                u[c] = *reinterpret_cast<const uint32_t*>(q);
+            }
         } else {
-            const uint8_t* c = w + rt * tile + ((kb / 4) * 64 + lane) * 16 + (kb % 4) * 4;
-            const int n = (e8 < 4 ? c[e8] : c[e8 - 4] >> 4) & 15;
-            return d * static_cast<float>((n ^ 8) - 8);
-        }
-    } else {
-        const uint8_t* b = w + o * row_bytes + kb * Fmt<WT>::kBytes;
-        const float d = HalfHw(*reinterpret_cast<const uint16_t*>(b));
-        if constexpr (WT == MLK_Q8_0) {
-            return d * static_cast<float>(static_cast<int8_t>(b[2 + e]));
-        } else if constexpr (WT == MLK_Q4_0) {
-            const int n = e < 16 ? b[2 + e] & 15 : b[2 + e - 16] >> 4;
-            return d * static_cast<float>(n - 8);
-        } else {
-            const int n = e < 16 ? b[4 + e] & 15 : b[4 + e - 16] >> 4;
-            return __fadd_rn(__fmul_rn(d, static_cast<float>(n)),
-                             HalfHw(*reinterpret_cast<const uint16_t*>(b + 2)));
+            const uint8_t* b = w + o * row_bytes + kb * Fmt<WT>::kBytes;
+            if constexpr (WT == MLK_Q4_1) {
+                d = *reinterpret_cast<const uint32_t*>(b);
+                u[0] = u[1] = *reinterpret_cast<const uint32_t*>(b + 4 + e);
+            } else {
+                d = *reinterpret_cast<const uint16_t*>(b);
+                u[0] = *reinterpret_cast<const u32_a2*>(b + 2 + e);
+                u[1] = WT == MLK_Q8_0 ? *reinterpret_cast<const u32_a2*>(b + 18 + e) : u[0];
+            }
         }
     }
-}
+    __device__ f32x4 Values(int c, int e) const {
+        const float s = HalfHw(d & 0xFFFFu);
+        // Q4: the nibbles of these inputs as bytes
+        uint32_t v = u[c];
+        if constexpr (WT == MLK_Q4_0 || WT == MLK_Q4_1) v = (v >> (4 * c)) & 0x0F0F0F0Fu;
+        if constexpr (WT == kWPlanarQ4) v = ((v >> e % 8) & 0x0F0F0F0Fu) ^ 0x08080808u;
+        f32x4 o;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t q = v >> (8 * i) & 0xFFu;
+            if constexpr (WT == MLK_Q4_1) {
+                o[i] = __fadd_rn(__fmul_rn(s, static_cast<float>(q)), HalfHw(d >> 16));
+            } else {
+                o[i] = s * static_cast<float>(WT == MLK_Q8_0 || WT == kWPlanarQ8
+                                                  ? static_cast<int>(static_cast<int8_t>(q))
+                                                  : static_cast<int>(q) - 8);
+            }
+        }
+        return o;
+    }
+};
+template <>
+struct Raw8<kWF32> {
+    f32x4 u[2];
+    __device__ void Load(const uint8_t* w, int64_t, int64_t, int64_t row_bytes, int64_t o,
+                         int64_t kb, int e) {
+        const float* p = reinterpret_cast<const float*>(w + o * row_bytes) + kb * 32 + e;
+        u[0] = *reinterpret_cast<const f32x4*>(p);
+        u[1] = *reinterpret_cast<const f32x4*>(p + 16);
+    }
+    __device__ f32x4 Values(int c, int) const { return u[c]; }
+};
 
 // ------------------------------------------------------------ the kernel
 // Epilogues.  kStore: y = sum + bias per segment, or partial sums; kAdd: y =
@@ -297,15 +384,17 @@ __device__ inline int At(int r, int g) { return r * 16 + ((g ^ ((r >> 1) & 3)) <
 
 // over the N lanes that hold one row
 template <int N>
-__device__ inline float RowSum(float v) {
-#pragma unroll
-    for (int m = 1; m < N; m *= 2) v += __shfl_xor(v, m, kWave);
-    return v;
-}
-template <int N>
 __device__ inline float RowMax(float v) {
 #pragma unroll
     for (int m = 1; m < N; m *= 2) v = fmaxf(v, __shfl_xor(v, m, kWave));
+    return v;
+}
+template <int N>
+__device__ inline uint32_t RowMin(uint32_t v) {
+#pragma unroll
+    for (int m = 1; m < N; m *= 2) {
+        v = min(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), m, kWave)));
+    }
     return v;
 }
 
@@ -313,45 +402,226 @@ __device__ inline f32x4 Mfma(h8 a, h8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
-// The outputs of marked rows (rinv 0) and, for split weights, of marked
-// outputs (cinv 0) of a tile: one thread an output, its inputs k0 .. k1 - 1
-// in order in fp32.
-template <int WT, int EPI, int BM, int BN>
-__device__ inline void SlowOutputs(const TileArgs& a, const TileSeg& g,
-                                                      const float* rinv, const float* cinv,
-                                                      int64_t m0, int64_t n0, int64_t k0,
-                                                      int64_t k1, float* out, int64_t ldo,
-                                                      bool bias) {
-    constexpr bool kDual = EPI == kSwiGlu;
-    constexpr int kCols = kDual ? BN / 2 : BN;
-    for (int e = threadIdx.x; e < BM * kCols; e += static_cast<int>(blockDim.x)) {
-        const int r = e / kCols, c = e % kCols;
-        const int64_t row = m0 + r, col = n0 + c;
-        if (row >= a.T || col >= g.rows) continue;
-        bool take = rinv[r] == 0.0f;
-        if constexpr (!kCodes<WT>) {
-            take = take || cinv[c] == 0.0f || (kDual && cinv[c + BN - kCols] == 0.0f);
-        }
-        if (!take) continue;
-        const auto sum = [&](const TileSeg& sg) {
-            float v = 0.0f;
-#pragma unroll 8
-            for (int64_t k = k0; k < k1; ++k) {
-                v = fmaf(a.x[row * a.K + k], Weight<WT>(sg.w, g.rows, a.K, a.row_bytes, col, k), v);
-            }
-            return v + (bias && sg.bias != nullptr ? sg.bias[col] : 0.0f);
+// Over the wave, in every lane.
+__device__ inline float WaveSum(float v) {
+#define MLK_DPP_ADD(ctrl, rows)                                                             \
+    v += __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_update_dpp(                 \
+        0, static_cast<int>(__float_as_uint(v)), ctrl, rows, 0xF, false)))
+    MLK_DPP_ADD(0xB1, 0xF);   // quad_perm 1 0 3 2
+    MLK_DPP_ADD(0x4E, 0xF);   // quad_perm 2 3 0 1
+    MLK_DPP_ADD(0x141, 0xF);  // row_half_mirror
+    MLK_DPP_ADD(0x140, 0xF);  // row_mirror
+    MLK_DPP_ADD(0x142, 0xA);  // row_bcast15 into rows 1, 3
+    MLK_DPP_ADD(0x143, 0xC);  // row_bcast31 into rows 2, 3
+#undef MLK_DPP_ADD
+    return __uint_as_float(static_cast<uint32_t>(
+        __builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(v)), 63)));
+}
+
+// The outputs n .. n + N - 1 of one marked row as fp32 products and sums: the
+// wave's lanes take consecutive blocks (their inputs in registers), every
+// output's sum is reduced over them and kept by one lane.
+template <int WT, int EPI, int N>
+__device__ inline void MarkedRow(const TileArgs& a, const TileSeg& g, int64_t row, int64_t n,
+                                 int64_t s0, int64_t s1, float* out, int64_t ldo, bool bias) {
+    constexpr int kMat = EPI == kSwiGlu ? 2 : 1;
+    const int lane = threadIdx.x & (kWave - 1);
+    float sum[kMat] = {};
+    for (int64_t z = s0; z < s1; z += kWave) {
+        // codes: the lane's block; fp32: its 4 inputs of every 256
+        const int64_t kb = z + lane < s1 ? z + lane : s1 - 1;
+        const auto at = [&](int i) {
+            if constexpr (WT != kWF32) return kb * kBK + 4 * i;
+            const int64_t k = z * kBK + 4 * kWave * i + 4 * lane;
+            return k < s1 * kBK ? k : s1 * kBK - 4;
         };
-        float* const o = out + row * ldo + col;
-        if constexpr (kDual) {
-            *o = SwiGluF(sum(g), sum(a.seg[1]));
-        } else {
-            *o = EPI == kAdd ? *o + sum(g) : sum(g);
+        const auto in = [&](int i) {
+            return WT == kWF32 ? z * kBK + 4 * kWave * i + 4 * lane < s1 * kBK : z + lane < s1;
+        };
+        f32x4 x[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            x[i] = *reinterpret_cast<const f32x4*>(a.x + row * a.K + at(i));
+        }
+        // G outputs' weights are loaded while the G before them are summed
+        constexpr int G = WT == kWF32 ? 1 : 4;
+        using LaneW = typename std::conditional<WT == kWF32, f32x4[8], Raw8<WT>[4]>::type;
+#pragma unroll
+        for (int p = 0; p < kMat; ++p) {
+            const uint8_t* const w = p == 0 ? g.w : a.seg[1].w;
+            LaneW lw[2][G];
+            const auto load = [&](int c0, LaneW (&l)[G]) {
+#pragma unroll
+                for (int c = 0; c < G; ++c) {
+                    const int64_t o = n + (c0 + c < N ? c0 + c : N - 1);
+                    const int64_t oc = o < g.rows ? o : g.rows - 1;
+                    if constexpr (WT == kWF32) {
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) {
+                            l[c][i] =
+                                *reinterpret_cast<const f32x4*>(w + oc * a.row_bytes + at(i) * 4);
+                        }
+                    } else {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            l[c][q].Load(w, g.rows, a.K, a.row_bytes, oc, kb, 4 * q);
+                        }
+                    }
+                }
+            };
+            const auto dot = [&](int c0, const LaneW (&l)[G]) {
+#pragma unroll
+                for (int c = 0; c < G; ++c) {
+                    float part = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) {
+                        f32x4 v;
+                        if constexpr (WT == kWF32) {
+                            v = l[c][i];
+                        } else {
+                            v = l[c][i % 4].Values(i / 4, 4 * (i % 4));
+                        }
+                        float t = 0.0f;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) t = fmaf(x[i][e], v[e], t);
+                        part += in(i) ? t : 0.0f;
+                    }
+                    part = WaveSum(part);
+                    if (lane == c0 + c) sum[p] += part;
+                }
+            };
+            load(0, lw[0]);
+            for (int c = 0; c < N; c += 2 * G) {
+                load(c + G, lw[1]);
+                dot(c, lw[0]);
+                load(c + 2 * G, lw[0]);
+                dot(c + G, lw[1]);
+            }
+        }
+    }
+    const int64_t col = n + lane;
+    if (lane >= N || col >= g.rows) return;
+    const float b0 = bias && g.bias != nullptr ? g.bias[col] : 0.0f;
+    float* const o = out + row * ldo + col;
+    if constexpr (kMat == 2) {
+        const float* const b1 = a.seg[1].bias;
+        *o = SwiGluF(sum[0] + b0, sum[1] + (b1 != nullptr ? b1[col] : 0.0f));
+    } else {
+        *o = EPI == kAdd ? *o + (sum[0] + b0) : sum[0] + b0;
+    }
+}
+
+// The marked outputs of a wave's rows m .. m + 16 MI - 1 (bit r of `rows`) and
+// outputs n .. n + 16 NB - 1 (bit c of `cols`: the output of every row) as
+// fp32 products and sums over blocks s0 .. s1 - 1, the operands straight from
+// memory, two blocks' loads at a time.  MFMA step st of 16 inputs from k on
+// multiplies inputs k + 4 kq + st.
+template <int WT, int EPI, int MI, int NB>
+__device__ inline void MarkedOutputs(const TileArgs& a, const TileSeg& g, uint64_t rows,
+                                     uint64_t cols, int64_t m, int64_t n, int64_t s0, int64_t s1,
+                                     float* out, int64_t ldo, bool bias) {
+    constexpr int kMat = EPI == kSwiGlu ? 2 : 1;
+    const int i16 = threadIdx.x & 15, kq = (threadIdx.x >> 4) & 3;
+    const float* xp[MI];
+    bool take[MI];
+    f32x4 e[MI][kMat][NB];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        take[i] = cols != 0 || ((rows >> (16 * i)) & 0xFFFFu) != 0;
+        const int64_t row = m + 16 * i + i16;
+        xp[i] = a.x + (row < a.T ? row : a.T - 1) * a.K + 4 * kq;
+#pragma unroll
+        for (int p = 0; p < kMat; ++p) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) e[i][p][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    if (rows == 0 && cols == 0) return;
+    for (int64_t z = s0; z < s1; z += 2) {
+        Raw8<WT> w[2][kMat][NB];
+        f32x4 x[2][MI][2];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int64_t kb = z + b < s1 ? z + b : z;
+#pragma unroll
+            for (int p = 0; p < kMat; ++p) {
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    const int64_t col = n + 16 * j + i16;
+                    w[b][p][j].Load(p == 0 ? g.w : a.seg[1].w, g.rows, a.K, a.row_bytes,
+                                    col < g.rows ? col : g.rows - 1, kb, 4 * kq);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < MI; ++i) {
+                if (!take[i]) continue;
+                x[b][i][0] = *reinterpret_cast<const f32x4*>(xp[i] + kb * kBK);
+                x[b][i][1] = *reinterpret_cast<const f32x4*>(xp[i] + kb * kBK + 16);
+            }
+        }
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            if (z + b >= s1) continue;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                f32x4 wv[kMat][NB];
+#pragma unroll
+                for (int p = 0; p < kMat; ++p) {
+#pragma unroll
+                    for (int j = 0; j < NB; ++j) wv[p][j] = w[b][p][j].Values(c, 4 * kq);
+                }
+#pragma unroll
+                for (int i = 0; i < MI; ++i) {
+                    if (!take[i]) continue;
+#pragma unroll
+                    for (int p = 0; p < kMat; ++p) {
+#pragma unroll
+                        for (int j = 0; j < NB; ++j) {
+#pragma unroll
+                            for (int st = 0; st < 4; ++st) {
+                                e[i][p][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                    x[b][i][c][st], wv[p][j][st], e[i][p][j], 0, 0, 0);
+                            }
+                        }
+                    }
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+        const int64_t col = n + 16 * j + i16;
+        if (col >= g.rows) continue;
+        const bool cb = (cols >> (16 * j + i16)) & 1;
+        const float b0 = bias && g.bias != nullptr ? g.bias[col] : 0.0f;
+        const float b1 = kMat == 2 && a.seg[1].bias != nullptr ? a.seg[1].bias[col] : 0.0f;
+#pragma unroll
+        for (int i = 0; i < MI; ++i) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t row = m + 16 * i + 4 * kq + r;
+                if (row >= a.T || !(cb || (rows >> (16 * i + 4 * kq + r) & 1))) continue;
+                float* const o = out + row * ldo + col;
+                if constexpr (EPI == kSwiGlu) {
+                    *o = SwiGluF(e[i][0][j][r] + b0, e[i][kMat - 1][j][r] + b1);
+                } else {
+                    *o = EPI == kAdd ? *o + (e[i][0][j][r] + b0) : e[i][0][j][r] + b0;
+                }
+            }
         }
     }
 }
 
+// Waves a SIMD that a workgroup's registers leave room for: three for the 64 x
+// 128 tiles of fp32 and Q4_1 weights, whose LDS fits a CU three times (F32, 64
+// rows of w_gate: 69.5 us with two, 66.3 with three; the 32 x 64 tiles, 8
+// rows: 50 us, 55 with their registers held to three).
+template <int WT, int BM>
+constexpr int kTileWaves = !kCodes<WT> && BM == 64 ? 3 : 2;
+
 template <int WT, int MI, int NJ, int WM, int WN, int EPI, int KB>
-__global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
+__global__ __launch_bounds__(64 * WM * WN,
+                             (kTileWaves<WT, 16 * MI * WM>)) void GemmTile(TileArgs a) {
     constexpr int kThreads = 64 * WM * WN;
     constexpr int BM = 16 * MI * WM, BN = 16 * NJ * WN;
     constexpr int kXN = BM * 4 / kThreads;    // 8-input groups of x per thread and stage
@@ -364,6 +634,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
     __shared__ Smem sm;
     __shared__ __align__(16) float rinv[BM];
     __shared__ float cinv[kCodes<WT> ? 4 : BN];
+    __shared__ uint32_t wlow;  // values: the weight rows' smallest scaled magnitude
     const int tile = static_cast<int>(blockIdx.x) % a.tiles;
     const int sp = static_cast<int>(blockIdx.x) / a.tiles;
     const int tm = tile % a.tiles_m, tn = tile / a.tiles_m;
@@ -449,29 +720,75 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
     };
     load(0, s0);
     load(1, s0 + 1 < s1 ? s0 + 1 : s0);
-    // the rows' scales, from their first 64 inputs
+    // the rows' scales, from their first 64 inputs: the thread's part of the
+    // two stages in registers
     PieceScale xs[kXN], wsc[kWN];
     float xmost[kXN], wmost[kWN];
+    uint32_t xleast[kXN], wleast[kWN];  // LeastKeys
+    us2 wkeys = {0xFFFF, 0xFFFF};       // Q4_1
+    const auto first_x = [&](int i) {
+        return RowMax<4>(AbsMax8(xv[1][i], AbsMax8(xv[0][i], 0.0f)));
+    };
+    const auto first_w = [&](int i) {
+        if constexpr (WT == kWF32) {
+            return RowMax<4>(AbsMax8(wr[1].v[i], AbsMax8(wr[0].v[i], 0.0f)));
+        } else if constexpr (WT == MLK_Q4_1) {
+            return fmaxf(BlockMost(wr[0]), BlockMost(wr[1]));
+        } else {
+            return 1.0f;
+        }
+    };
+    bool none = false;
 #pragma unroll
     for (int i = 0; i < kXN; ++i) {
-        xs[i] = PieceScale(RowSum<4>(AbsSum8(xv[0][i]) + AbsSum8(xv[1][i])) * (1.0f / 64.0f));
-        xmost[i] = 0.0f;
+        xmost[i] = first_x(i);
+        none |= xmost[i] == 0.0f;
     }
 #pragma unroll
     for (int i = 0; i < kWN; ++i) {
-        wmost[i] = 0.0f;
-        if constexpr (WT == kWF32) {
-            wsc[i] = PieceScale(RowSum<4>(AbsSum8(wr[0].v[i]) + AbsSum8(wr[1].v[i])) *
-                                (1.0f / 64.0f));
-        } else if constexpr (WT == MLK_Q4_1) {
-            float4 e[2][2], f[2][2];
-            Values16(wr[0], h, e);
-            Values16(wr[1], h, f);
-            wsc[i] = PieceScale(RowSum<2>((AbsSum8(e[0]) + AbsSum8(e[1])) +
-                                          (AbsSum8(f[0]) + AbsSum8(f[1]))) *
-                                (1.0f / 64.0f));
-        }
+        wmost[i] = first_w(i);
+        none |= wmost[i] == 0.0f;
     }
+    if (__any(none)) {  // rows that begin with zeros: 64 inputs at 7 places further on
+        for (int k = 1; k < 8 && __any(none); ++k) {
+            const int64_t z = s0 + (s1 - s0) * k / 8;
+            load(0, z);
+            load(1, z + 1 < s1 ? z + 1 : z);
+            none = false;
+#pragma unroll
+            for (int i = 0; i < kXN; ++i) {
+                const float m = first_x(i);
+                if (xmost[i] == 0.0f) xmost[i] = m;
+                none |= xmost[i] == 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < kWN; ++i) {
+                const float m = first_w(i);
+                if (wmost[i] == 0.0f) wmost[i] = m;
+                none |= wmost[i] == 0.0f;
+            }
+        }
+        load(0, s0);
+        load(1, s0 + 1 < s1 ? s0 + 1 : s0);
+    }
+#pragma unroll
+    for (int i = 0; i < kXN; ++i) {
+        xs[i] = PieceScale(xmost[i], 7);
+        xmost[i] = 0.0f;
+        xleast[i] = kNoKey;
+    }
+#pragma unroll
+    for (int i = 0; i < kWN; ++i) {
+        wsc[i] = PieceScale(wmost[i], 10);
+        wmost[i] = 0.0f;
+        wleast[i] = kNoKey;
+    }
+
+    // LDS offsets of the thread's writes and operand reads; rows a multiple of
+    // 8 apart have the same swizzle, so the others lie constants away
+    const int xw = At(tid >> 2, tid & 3);
+    const int ww = WT == kWF32 ? xw : At(tid >> 1, 2 * h), ww1 = At(tid >> 1, 2 * h + 1);
+    const int xr = wm * 256 * MI + At(i16, kq), wrd = wn * 256 * NJ + At(i16, kq);
 
     // a stage's registers b into LDS buffer buf
     auto store = [&](int buf, int b) {
@@ -480,30 +797,37 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
         for (int i = 0; i < kXN; ++i) {
             Split8(xv[b][i], xs[i].s, &p0, &p1);
             xmost[i] = AbsMax8(xv[b][i], xmost[i]);
-            const int at = At((tid >> 2) + kThreads / 4 * i, tid & 3);
+            xleast[i] = LeastKey8(xv[b][i], xleast[i]);
+            const int at = xw + kThreads * 4 * i;
             *reinterpret_cast<u32x4*>(&sm.x[buf][0][at]) = p0;
             *reinterpret_cast<u32x4*>(&sm.x[buf][1][at]) = p1;
         }
         if constexpr (kCodes<WT>) {
             u32x4 c[2];
             Codes16<WT>(wr[b], h, c);
-            *reinterpret_cast<u32x4*>(&sm.w[buf][0][At(tid >> 1, 2 * h)]) = c[0];
-            *reinterpret_cast<u32x4*>(&sm.w[buf][0][At(tid >> 1, 2 * h + 1)]) = c[1];
+            *reinterpret_cast<u32x4*>(&sm.w[buf][0][ww]) = c[0];
+            *reinterpret_cast<u32x4*>(&sm.w[buf][0][ww1]) = c[1];
             sm.d[buf][tid >> 1] = HalfHw(wr[b].d & 0xFFFFu);
         } else {
             float4 q[2][2];
-            if constexpr (WT == MLK_Q4_1) Values16(wr[b], h, q);
+            if constexpr (WT == MLK_Q4_1) {
+                Values16(wr[b], h, q);
+                wmost[0] = fmaxf(wmost[0], BlockMost(wr[b]));
+                wkeys = __builtin_elementwise_min(wkeys, BlockKeys(wr[b]));
+            }
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
+                const int k = WT == kWF32 ? i : 0;
                 if constexpr (WT == kWF32) {
                     q[i][0] = wr[b].v[i][0];
                     q[i][1] = wr[b].v[i][1];
                 }
-                const int k = WT == kWF32 ? i : 0;
                 Split8(q[i], wsc[k].s, &p0, &p1);
-                wmost[k] = AbsMax8(q[i], wmost[k]);
-                const int at = WT == kWF32 ? At((tid >> 2) + BN / 2 * i, tid & 3)
-                                           : At(tid >> 1, 2 * h + i);
+                if constexpr (WT == kWF32) {
+                    wmost[i] = AbsMax8(q[i], wmost[i]);
+                    wleast[i] = LeastKey8(q[i], wleast[i]);
+                }
+                const int at = WT == kWF32 ? ww + BN * 8 * i : (i == 0 ? ww : ww1);
                 *reinterpret_cast<u32x4*>(&sm.w[buf][0][at]) = p0;
                 *reinterpret_cast<u32x4*>(&sm.w[buf][kPl - 1][at]) = p1;
             }
@@ -523,6 +847,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
     // block, one barrier.
     auto step = [&](int64_t s, int u) {
         h8 b[KB][kPl][NJ];
+        h8 bl[KB][NJ];  // codes for the second pieces, times 2^-11
         float dj[KB][NJ];
 #pragma unroll
         for (int k = 0; k < KB; ++k) {
@@ -533,9 +858,12 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
                 const int row = wn * 16 * NJ + 16 * j + i16;
 #pragma unroll
                 for (int p = 0; p < kPl; ++p) {
-                    b[k][p][j] = *reinterpret_cast<const h8*>(&sm.w[buf][p][At(row, kq)]);
+                    b[k][p][j] = *reinterpret_cast<const h8*>(&sm.w[buf][p][wrd + 256 * j]);
                 }
-                if constexpr (kCodes<WT>) dj[k][j] = sm.d[buf][row];
+                if constexpr (kCodes<WT>) {
+                    bl[k][j] = b[k][0][j] * static_cast<_Float16>(1.0f / kLowUp);
+                    dj[k][j] = sm.d[buf][row];
+                }
             }
         }
 #pragma unroll
@@ -547,7 +875,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
                 if constexpr (KB == 2) load(i / kh, s + 4 + i / kh < s1 ? s + 4 + i / kh : s1 - 1);
             }
             h8 hi[KB], lo[KB];
-            const int at = At(wm * 16 * MI + 16 * i + i16, kq);
+            const int at = xr + 256 * i;
 #pragma unroll
             for (int k = 0; k < KB; ++k) {
                 hi[k] = *reinterpret_cast<const h8*>(&sm.x[KB * u + k][0][at]);
@@ -559,7 +887,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
                 for (int k = 0; k < KB; ++k) {
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) {
-                        S[k][j] = Mfma(lo[k], b[k][0][j], f32x4{0.f, 0.f, 0.f, 0.f});
+                        S[k][j] = Mfma(lo[k], bl[k][j], f32x4{0.f, 0.f, 0.f, 0.f});
                     }
 #pragma unroll
                     for (int j = 0; j < NJ; ++j) S[k][j] = Mfma(hi[k], b[k][0][j], S[k][j]);
@@ -576,17 +904,30 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
                     }
                 }
             } else {
+                f32x4 S[NJ];  // the products with a second piece, times 2^11
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = Mfma(lo[0], b[0][0][j], acc[i][j]);
+                for (int j = 0; j < NJ; ++j) {
+                    S[j] = Mfma(lo[0], b[0][0][j], f32x4{0.f, 0.f, 0.f, 0.f});
+                }
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) acc[i][j] = Mfma(hi[0], b[0][kPl - 1][j], acc[i][j]);
+                for (int j = 0; j < NJ; ++j) S[j] = Mfma(hi[0], b[0][kPl - 1][j], S[j]);
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) acc[i][j] = Mfma(hi[0], b[0][0][j], acc[i][j]);
+#pragma unroll
+                for (int j = 0; j < NJ; ++j) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        acc[i][j][r] = fmaf(S[j][r], 1.0f / kLowUp, acc[i][j][r]);
+                    }
+                }
             }
         }
         __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
     };
+    if constexpr (!kCodes<WT>) {
+        if (tid == 0) wlow = 0x7F800000u;
+    }
     store(0, 0);
     if constexpr (KB == 2) {
         store(1, 1);
@@ -602,36 +943,48 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
     if (s < s1) step(s, 0);
 
     // the factors that undo the scales; 0 marks a row whose values leave the
-    // pieces' range
+    // pieces' range (head comment)
+    const float low_min = 1.0f / ((kCodes<WT> ? 2048.0f : 1024.0f) * static_cast<float>(a.K));
+    const float low_pair = 1.0f / (33554432.0f * static_cast<float>(a.K));
     bool bad = false;
-#pragma unroll
-    for (int i = 0; i < kXN; ++i) {
-        const float inv = xs[i].Checked(RowMax<4>(xmost[i]));
-        rinv[(tid >> 2) + kThreads / 4 * i] = inv;
-        bad |= inv == 0.0f;
-    }
+    float low = INFINITY;  // values: the smallest scaled weight of the tile
     if constexpr (!kCodes<WT>) {
 #pragma unroll
         for (int i = 0; i < kWN; ++i) {
-            const float inv = wsc[i].Checked(RowMax<WT == kWF32 ? 4 : 2>(wmost[i]));
-            cinv[WT == kWF32 ? (tid >> 2) + BN / 2 * i : tid >> 1] = inv;
-            bad |= inv == 0.0f;
+            const float most = WT == kWF32 ? RowMax<4>(wmost[i]) : wmost[i];
+            const float least =
+                WT == kWF32 ? KeyValue(RowMin<4>(wleast[i])) : KeySpacing(wkeys);
+            const bool fits = wsc[i].Fits(most, least, low_min);
+            cinv[WT == kWF32 ? (tid >> 2) + BN / 2 * i : tid >> 1] = fits ? wsc[i].inv : 0.0f;
+            bad |= !fits;
+            if (fits) low = fminf(low, least * wsc[i].s);
         }
+        atomicMin(&wlow, __float_as_uint(low));
+        __syncthreads();
+        low = __uint_as_float(wlow);
+    }
+#pragma unroll
+    for (int i = 0; i < kXN; ++i) {
+        const float least = KeyValue(RowMin<4>(xleast[i]));
+        bool fits = xs[i].Fits(RowMax<4>(xmost[i]), least, low_min);
+        if constexpr (!kCodes<WT>) fits = fits && !(least * xs[i].s * low < low_pair);
+        rinv[(tid >> 2) + kThreads / 4 * i] = fits ? xs[i].inv : 0.0f;
+        bad |= !fits;
     }
     const bool any_bad = __syncthreads_or(bad) != 0;
 
     const bool part = a.partial != nullptr;
     const int64_t ldo = part ? a.cols : O;
     float* const out = part ? a.partial + sp * a.T * a.cols + g.col0 : (kDual ? a.seg[1].y : g.y);
+    const auto factors = [&](int i) {
+        return *reinterpret_cast<const f32x4*>(&rinv[wm * 16 * MI + 16 * i + 4 * kq]);
+    };
     const auto value = [&](int i, int j, int r, float ri) {
         if constexpr (kCodes<WT>) {
             return acc[i][j][r] * ri;
         } else {
             return acc[i][j][r] * (ri * cinv[wn * 16 * NJ + 16 * j + i16]);
         }
-    };
-    const auto factors = [&](int i) {
-        return *reinterpret_cast<const f32x4*>(&rinv[wm * 16 * MI + 16 * i + 4 * kq]);
     };
     if constexpr (kDual) {
         // The stage buffers are free.  Gate wave (wm, wn) and up wave
@@ -708,29 +1061,63 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void GemmTile(TileArgs a) {
             }
         }
     }
-    if (any_bad) {
-        SlowOutputs<WT, EPI, BM, BN>(a, g, rinv, cinv, m0, n0, s0 * kBK, s1 * kBK, out, ldo, !part);
+    if (__builtin_expect(any_bad, 0)) {
+        // up to 8 marked rows one by one, each wave a part of the outputs;
+        // more, and marked outputs, by the matrix cores, each wave its rows
+        // and, of the tile's outputs, 1 / WN
+        constexpr int NB = kDual ? NJ / 2 : NJ;
+        const auto marked = [](const float* f, int n, int l) {
+            return __ballot(l < n && f[l < n ? l : 0] == 0.0f);
+        };
+        uint64_t all_rows[WM];
+        int n_rows = 0;
+#pragma unroll
+        for (int i = 0; i < WM; ++i) {
+            const int64_t left = a.T - m0 - 16 * MI * i;  // (rows past T are copies of the last)
+            all_rows[i] = marked(rinv + 16 * MI * i,
+                                 left < 16 * MI ? static_cast<int>(left) : 16 * MI, lane);
+            n_rows += __popcll(all_rows[i]);
+        }
+        bool any_col = false;
+        uint64_t cols = 0;
+        if constexpr (!kCodes<WT>) {
+            for (int i = 0; i < BN; i += kWave) any_col |= marked(cinv + i, kWave, lane) != 0;
+            const float* const f = cinv + wn * 16 * NB;
+            cols = marked(f, 16 * NB, lane);
+            if (kDual) cols |= marked(f + BN / 2, 16 * NB, lane);
+        }
+        if (n_rows <= 8 && !any_col) {
+            constexpr int N = (kDual ? BN / 2 : BN) / (WM * WN);
+#pragma unroll
+            for (int i = 0; i < WM; ++i) {
+                for (uint64_t b = all_rows[i]; b != 0; b &= b - 1) {
+                    const int64_t row = m0 + 16 * MI * i + __builtin_ctzll(b);
+                    MarkedRow<WT, EPI, N>(a, g, row, n0 + wave * N, s0, s1, out, ldo, !part);
+                }
+            }
+        } else {
+            MarkedOutputs<WT, EPI, MI, NB>(a, g, all_rows[wm], cols, m0 + wm * 16 * MI,
+                                           n0 + wn * 16 * NB, s0, s1, out, ldo, !part);
+        }
     }
 }
-
 
 // ------------------------------------------------------------ launches
 // Tile shape and K splits of a launch.
 //   128 x 256 (one workgroup a CU) for more than 64 rows, where up to 8
 //       splits (more while each keeps 16 stages) give 3/4 of a workgroup a
 //       CU; past that K is not split: T = 389 over 14336 outputs (224 tiles,
-//       Q8_0) took 150 us unsplit, 176 us in two splits of 1.75 rounds.
+//       Q8_0) takes 160 us unsplit, 17% more in two splits of 1.75 rounds.
 //   32 x 64 up to 32 rows, split to 4 workgroups a CU (33 KB of LDS each),
-//       each split at least 8 stages.  16 rows of F32: w_gate 52 us (fp32
-//       MFMA 52), wo 19.9 (20.2); 32 rows of Q8_0 / Q4_0: w_gate 42 / 40 us
-//       (skinny kernel, fp32 MFMA, 48 / 47), 128256 outputs 263 / 216 (355 /
-//       366, whose 8 splits' partial sums alone are 131 MB).  On 64 x 128
-//       tiles the same take 46, 21.7, 40 / 39 and 265 / 228, Q8_0 wo 22 (19.3
-//       here).
+//       each split at least 8 stages.  16 rows of F32: w_gate 50.6 us (fp32
+//       MFMA 51.2); 32 rows of Q8_0 / Q4_0: w_gate 41.7 / 40.5 us (skinny
+//       kernel, fp32 MFMA, 49.5 / 48.4), 128256 outputs 273 / 222 (350 / 360,
+//       whose 8 splits' partial sums alone are 131 MB).  On 64 x 128 tiles
+//       those took as long or longer.
 //   64 x 128 otherwise, split to 1.5 workgroups a CU, each split at least 8
-//       stages.  Q8_0: T = 64 over 4096 x 14336 39.6 us in 16 splits (512
-//       workgroups), 46 in 8; 128 rows over 4096 x 4096 31 us against 34-37
-//       on 128 x 256, over 14336 x 4096 70 against 55.
+//       stages.  Q8_0: T = 64 over 4096 x 14336 43 us in 16 splits (512
+//       workgroups), 16% more in 8; 128 rows over 4096 x 4096 31 us against
+//       34-37 on 128 x 256, over 14336 x 4096 61 there against 70.
 // Measured beside these: 128 x 128 tiles (4 waves) 7-14% slower than 128 x
 // 256 at every T from 200 to 4096.
 struct TilePlan {
@@ -858,7 +1245,8 @@ bool TileChosen(int wt, int64_t T, int64_t K, int64_t cols, bool fused) {
     if (T > 32) return true;
     const int64_t n = K * cols;
     if (wt == kWF32) return T >= 8 || (T >= 5 && n >= kFewRowsMin);
-    return (wt == MLK_Q8_0 || wt == MLK_Q4_0) && T > 16 && n >= (fused ? kLayerGroupMin : kFewRowsMin);
+    return (wt == MLK_Q8_0 || wt == MLK_Q4_0) && T > 16 &&
+           n >= (fused ? kLayerGroupMin : kFewRowsMin);
 }
 
 bool TileWeightAligned(int wt, const void* w) {

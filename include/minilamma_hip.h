@@ -208,9 +208,10 @@ mlk_status mlk_quant_to_planar(int32_t quant_type, const void* blocks, int64_t r
  * matrix cores with exact products (codes are exact in bf16 and x is split
  * into three exact bf16 pieces), and need a workspace of
  * mlk_linear_planar_workspace_bytes (16-byte aligned); more rows take the
- * tiled matrix-core GEMM (x in two fp16 pieces under a power of two per row,
- * each value to within one unit of its fp32 last place; rows outside the
- * pieces' range in fp32), with the optional workspace of
+ * tiled matrix-core GEMM (x in two fp16 pieces under a power of two per row:
+ * each product to within 2^-22 of itself, for inputs 2^(18 + log2
+ * in_features) below the row's first ones to within in_features * 2^-25; rows
+ * of more range in fp32), with the optional workspace of
  * mlk_linear_workspace_bytes.  No counterpart in the reference. */
 mlk_status mlk_linear_planar(int32_t quant_type, const float* x, const void* w_planar,
                              const float* bias, float* y, int64_t rows, int64_t in_features,

@@ -5,9 +5,12 @@ below 8 rows.
 
 Bar: every output within gamma_K * sum_k |x_k w_k| of the float64 product
 with the dequantized weights (conftest.assert_dot_close).  A product here is
-within 3 * 2^-22 of its exact value (each operand to one unit of its last of
-23 bits, the product of the two low pieces left out), 12 u; with K >= 256 and
-one fp32 rounding per 32 inputs and piece the sums stay below K u."""
+within 12 u of its exact value (two pieces of an operand hold it to 2^-23, the
+product of the two low pieces, below 2^-22, is left out), more only for
+values more than 2^(18 + log2 K) below the largest of their row's first
+inputs, and within K / 2 u (F32, Q4_1: 5 K / 4 u) down to the bounds of the
+pieces' range, where rows are summed in fp32; the sums' own errors stay far
+below K u, with one fp32 rounding per 32 inputs and piece."""
 from __future__ import annotations
 
 import numpy as np
@@ -109,6 +112,105 @@ def test_tile_row_scales(mlk, orc, kind, T):
     err = np.abs(got[ok].astype(np.float64) - ex)
     lim = K * u / (1 - K * u) * s + 1e-44
     assert (err[fits] <= lim[fits]).all(), f"{kind}: {int((err > lim)[fits].sum())} outside"
+
+
+# (kind, out, in, rows): all types above 32 rows (64- and 128-row tiles, an odd
+# number of blocks), and the 32-row tiles
+WIDE = [(k, 300, K, T) for k in TYPES for K, T in ((512, 40), (4096, 130))] + [
+    ("f32", 130, 544, 9), ("q4_1", 130, 544, 33), ("q8_0", 32769, 1056, 17),
+    ("f32", 260, 288, 200), ("q4_0", 257, 288, 200)]
+
+
+def bar(kind, got, x, wd, what):
+    ex, s = dot_exact(x, wd)
+    u, K = 2.0 ** -24, x.shape[1]
+    over = np.abs(got.astype(np.float64) - ex) / (K * u / (1 - K * u) * s + 1e-44)
+    assert over.max() <= 1, f"{kind} {what}: {over.max():.3g} times the bar"
+
+
+@pytest.mark.parametrize("kind,out,K,T", WIDE)
+def test_tile_large_inputs_meet_zero_weights(mlk, orc, kind, out, K, T):
+    """Large values among a row's first inputs (where its scale is taken) or
+    anywhere whose products vanish: every other value keeps its precision.
+    For fp32 and Q4_1 weights also the mirror, large weights over zero
+    inputs."""
+    rng = np.random.default_rng(K + T)
+    B = 64  # whole blocks of zero weights: their codes' values are exact zeros
+    for big in (1e4, 1e6, 1e8, 1e10, 1e15, 1e25):
+        x, w = normal(rng, (T, K)), normal(rng, (out, K), 0.02)
+        w[:, :B] = w[:, K - 32:] = 0
+        x[::3, 5] = big
+        x[1::3, :B] = big
+        x[2::9, K - 7] = big  # (the others of 2::3: no large value)
+        got, wd = run(mlk, orc, kind, x, w)
+        bar(kind, got, x, wd, f"x {big:g}")
+        if kind == "f32" or (kind == "q4_1" and big <= 1e4):  # fp16 block scales
+            x, w = normal(rng, (T, K)), normal(rng, (out, K), 1e-3 if kind == "q4_1" else 0.02)
+            x[:, :B] = x[:, K - 32:] = 0
+            w[::3, 5] = big
+            w[1::3, :B] = big
+            w[2::9, K - 7] = big
+            got, wd = run(mlk, orc, kind, x, w)
+            bar(kind, got, x, wd, f"w {big:g}")
+
+
+@pytest.mark.parametrize("kind", TYPES)
+@pytest.mark.parametrize("K,T,count", [(256, 40, 1), (512, 200, 3), (1024, 130, 40), (256, 300, 300)])
+def test_tile_few_small_values(mlk, orc, kind, K, T, count):
+    """Tiny values among ordinary ones, picked alone by weights of one 1 each:
+    in few rows of a tile (summed one by one) and in all.  For fp32 weights
+    also tiny weights under inputs of one 1 each, and both at once."""
+    rng = np.random.default_rng(K + count)
+
+    def dot(m, rows):
+        for r in rows:
+            at = rng.choice(K, min(count, K), replace=False)
+            m[r, at] *= (10.0 ** rng.uniform(-15, -6, len(at))).astype(np.float32)
+    x = normal(rng, (T, K))
+    dot(x, range(T) if count == 300 else range(3, T, 29))
+    w = np.zeros((K, K), np.float32)
+    w[np.arange(K), rng.permutation(K)] = 1
+    got, wd = run(mlk, orc, kind, x, w)
+    bar(kind, got, x, wd, "x")
+    if kind != "f32":
+        return
+    w = normal(rng, (K, K), 0.02)
+    dot(w, range(5, K, 31))
+    e = np.zeros((T, K), np.float32)
+    e[np.arange(T), rng.integers(0, K, T)] = 1
+    got, _ = run(mlk, orc, kind, e, w)
+    bar(kind, got, e, w, "w")
+    # both: x's and w's tiny values at the same inputs, the others meet zeros
+    x, w = normal(rng, (T, K)), normal(rng, (K, K))
+    x[:, :K // 2] = 0
+    w[:, K // 2:] = 0
+    at = rng.choice(K, 5, replace=False)
+    x[3::29, at] = (10.0 ** rng.uniform(-12, -5, (len(x[3::29]), 5))).astype(np.float32)
+    w[::17, at] = (10.0 ** rng.uniform(-12, -5, (len(w[::17]), 5))).astype(np.float32)
+    got, _ = run(mlk, orc, kind, x, w)
+    bar(kind, got, x, w, "both")
+
+
+@pytest.mark.parametrize("K,T", [(256, 40), (512, 200), (1056, 9)])
+def test_tile_sparse_and_small(mlk, orc, K, T):
+    """fp32 weights that pick single inputs (a permutation), with inputs of
+    every magnitude, and outputs that consist of products of small values
+    alone, each side's large values meeting zeros."""
+    rng = np.random.default_rng(K)
+    x = (normal(rng, (T, K)) * 10.0 ** rng.uniform(-9, 3, (T, K))).astype(np.float32)
+    w = np.zeros((K, K), np.float32)
+    w[np.arange(K), rng.permutation(K)] = 1
+    got, _ = run(mlk, orc, "f32", x, w)
+    bar("f32", got, x, w, "permutation")
+    third = K // 3
+    for e in range(-40, 1, 4):
+        x, w = normal(rng, (T, K)), normal(rng, (300, K))
+        w[:, :third] = 0
+        x[:, third:2 * third] = 0
+        x[:, 2 * third:] *= 2.0 ** e
+        w[:, 2 * third:] *= 2.0 ** e
+        got, _ = run(mlk, orc, "f32", x, w)
+        bar("f32", got, x, w, f"2^{e}")
 
 
 @pytest.mark.parametrize("wt", ["q8_0", "q4_1", "f32"])
