@@ -844,17 +844,17 @@ GEMM_TOKENS = (8, 16, 32, 64, 128, 512, 4096)
 MFMA_FP32_PEAK_TFLOPS = 157.3  # MI355X dense fp32 matrix-core peak
 MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16 matrix-core peak
 MFMA_FP16_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS  # the same rate
-# The tiled GEMM (more than 32 token rows) and the attention at head_dim 128
-# split values into two fp16 pieces: two fp16 MACs per useful MAC over Q8_0 /
-# Q4_0 codes, three over fp32 or Q4_1 weights and in the attention.
+# The tiled GEMM (more than 32 token rows) splits values into two fp16 pieces:
+# two fp16 MACs per useful MAC over Q8_0 / Q4_0 codes, three over fp32 or Q4_1
+# weights; the attention at head_dim 128 into three exact bf16 pieces.
 
 
 def attention_peak(hd):
     """(peak TFLOP/s of useful MACs, basis) of the tile attention: at
-    head_dim 128 the scores and the values each take 3 fp16 piece products
+    head_dim 128 the scores and the values each take 6 bf16 piece products
     per useful MAC, at 64 the fp32 instruction."""
     if hd == 128:
-        return MFMA_FP16_PEAK_TFLOPS / 3, "fp16 MFMA / 3 (piece products)"
+        return MFMA_BF16_PEAK_TFLOPS / 6, "bf16 MFMA / 6 (piece products)"
     return MFMA_FP32_PEAK_TFLOPS, "fp32 MFMA"
 
 
@@ -1645,7 +1645,7 @@ def kernel_summary(out_md, title, bench_json, kt_dir, fetch_dir=None, write_dir=
            "launches -- for --linear, around one replay of a HIP graph holding each "
            "projection's calls, so the figure is kernel time, not Python dispatch; HBM-bound "
            "cases on rotating cold copies, against 8 TB/s; "
-           "matrix-core cases against the peak of the instruction they run: 157.3 TFLOP/s fp32 MFMA, or for fp16 piece products the 2.5 PFLOP/s fp16 peak over the fp16 MACs per useful MAC, 2 over Q8_0 / Q4_0 codes and 3 over fp32 and Q4_1 weights and in the attention):", "",
+           "matrix-core cases against the peak of the instruction they run: 157.3 TFLOP/s fp32 MFMA, or for piece products the 2.5 PFLOP/s fp16 and bf16 peak over the MACs per useful MAC, 2 over Q8_0 / Q4_0 codes, 3 over fp32 and Q4_1 weights and 6 in the attention):", "",
            "| case | us | throughput | fraction of peak |", "|---|---|---|---|"]
 
     def rate(node, prefix=""):

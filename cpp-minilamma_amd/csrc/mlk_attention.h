@@ -15,29 +15,29 @@ bool PrefillSupported(int32_t head_dim, const float* q, int64_t q_row_stride, co
 // 0 .. pos0 + t; kc / vc point at the layer's [max_seq, KV, head_dim] slice,
 // slot = KV * head_dim floats per position.  Arguments already validated.
 // With a 16-byte aligned workspace of PrefillImageBytes(KV, head_dim,
-// pos0 + T) bytes (head_dim 128, T >= kPrefillImageMinTokens), K and V of
-// positions 0 .. pos0 + T - 1 are first split into fp16 piece images, one
-// launch, which the tiles then copy instead of splitting each tile in every
-// workgroup; the sums are the same.  Otherwise no workspace is used.  Below
-// that many tokens a tile is staged by too few workgroups for the extra
-// launch to pay (Llama-3-8B heads, from position 0: 128 tokens 14.8 -> 14.1
-// us with the images, 64 tokens 10.0 -> 10.9; 389 tokens at 1500: 133 -> 96,
-// 4096 tokens 629 -> 483).  a_planes (16-byte aligned, H * head_dim a
-// multiple of 32), when set, also receives the output rows as StorePlanes
-// planes.
-constexpr int64_t kPrefillImageMinTokens = 128;
+// pos0 + T) bytes (head_dim 128, PrefillImages), K and V of positions 0 ..
+// pos0 + T - 1 are first split into bf16 piece images, one launch, which the
+// tiles then copy instead of splitting each tile in every workgroup; the sums
+// are the same.  Otherwise no workspace is used.  a_planes (16-byte aligned,
+// H * head_dim a multiple of 32), when set, also receives the output rows as
+// StorePlanes planes.
+// Where the images pay: a tile has to be staged by enough workgroups (Llama-3
+// heads, 8B / 70B: 389 tokens after 1500 133 -> 124 / 169 -> 162 us, at 4000
+// in chunks 229 -> 221, 128 tokens there 77 -> 83, 1024 from position 0 80 ->
+// 77 / 118 -> 114, 4096 763 -> 708 / 1547 -> 1427, but 512 41 -> 40 / 44 ->
+// 47).
+inline bool PrefillImages(int64_t T, int64_t pos0) { return T >= 1024 || (T >= 384 && pos0 >= T); }
 // A prompt chunk whose token blocks are at most one workgroup per compute
 // unit, over a context of at least kPrefillSplitMinCtx positions, is split
 // over chunks of positions like decode tokens (LaunchDecodeTile): the number
 // of chunks of its n_pos positions (1: not split; at most TileChunk's for
 // max_ctx) and their length.  Llama-3-8B heads, whole ->
-// in chunks: 64 tokens at 4000 277 -> 42 us, 128 at 4000 197 -> 66, 389 at
-// 6000 303 -> 220; more blocks than units fill the chip by themselves (700 at
-// 2000: 154 whole, 233 in chunks).  Over short contexts the merge costs more
-// than the split gives (389 from position 0: 27 whole, 55 in chunks); over
-// 1000 positions it would gain (128 tokens 61 -> 39), but up to here a
-// call with a workspace keeps the sums of the prefill entry, which has none,
-// bit for bit.
+// in chunks: 64 tokens at 4000 267 -> 47 us, 128 at 4000 278 -> 77, 389 at
+// 6000 424 -> 328; more blocks than units fill the chip by themselves (700 at
+// 2000 took 1.5 times as long in chunks).  Over short contexts the merge costs
+// more than the split gives (389 from position 0 took twice as long); over
+// 1000 positions it would gain (128 tokens a third), but up to here a call with
+// a workspace keeps the sums of the prefill entry, which has none, bit for bit.
 constexpr int64_t kPrefillSplitMinCtx = 2048;
 int64_t PrefillChunks(int64_t T, int32_t H, int32_t KV, int64_t n_pos, int64_t max_ctx,
                       int* chunk);

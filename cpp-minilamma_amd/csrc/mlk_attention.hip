@@ -859,7 +859,7 @@ int64_t PromptAttentionBytes(int64_t T, int32_t H, int32_t KV, int32_t head_dim,
     int chunk = 0;
     const int64_t nc = PrefillChunks(T, H, KV, max_ctx, max_ctx, &chunk);
     int64_t b = nc > 1 ? (PartialBytes(T, H, nc, head_dim) + 255) / 256 * 256 : 0;
-    if (T >= kPrefillImageMinTokens) b += PrefillImageBytes(KV, head_dim, max_ctx);
+    if (PrefillImages(T, max_ctx - T)) b += PrefillImageBytes(KV, head_dim, max_ctx);
     return b;
 }
 
@@ -951,7 +951,7 @@ mlk_status AttentionDecode(const float* q, int64_t q_row_stride, const float* k_
         const int64_t images = (need + 255) / 256 * 256;
         const int64_t image_bytes =
             prompt_split ? PrefillImageBytes(n_kv_heads, head_dim, pos0 + n_tokens) : 0;
-        void* images_at = image_bytes > 0 && n_tokens >= kPrefillImageMinTokens &&
+        void* images_at = image_bytes > 0 && PrefillImages(n_tokens, pos0) &&
                                   static_cast<int64_t>(workspace_bytes) >= images + image_bytes
                               ? static_cast<char*>(workspace) + images
                               : nullptr;

@@ -32,29 +32,25 @@
 // per KV head that are not a multiple of 4) computes on head 0's query and
 // stores nothing: no branch around the loop body.  FLOPs: 4 * hd * H * sum_t (pos0 + t + 1).
 //
-// fp16 products (kF16: every launch at head_dim 128; head_dim 64 keeps the
-// fp32 instruction above): K, V, q and p are each scaled by a power of two and
-// split into two fp16 pieces, the value rounded to fp16 and the rest rounded
-// to fp16 (together within one unit of its last of 23 bits; for values far
-// below their tile's largest, within 2^-39 of that).  The scale comes from the
-// largest finite magnitude of a K tile, of a V tile (32 positions x 128 dims)
-// and of a q row, which it brings into [2^14, 2^15); p, at most 1, is scaled by
-// 2^14 and by the V tile's factor relative to the largest so far, so the
-// accumulators keep one unit.  Each product is lo hi + hi lo + hi hi, three
-// v_mfma_f32_16x16x32_f16 (32 dims or the tile's 32 positions each); lo lo,
-// below 2^-22, is left out.  Six bf16 piece products (three pieces a value)
-// took twice the matrix work and half as much LDS again: Llama-3-8B heads,
-// 4096 tokens from position 0, 721 us before, 484 with these (284 TFLOP/s of
-// q.k and p.v), error against float64 1.6e-7 before, 1.2e-7 after; 64 decode
-// tokens over 1000 positions 66 -> 62 us.  Scores stay within
-// the gamma_{hd+1} bound with the fp32 sums; values add at most 16 u of
-// sum_j p_j |v_jd| to the sums' (n + 6) u.
-// Tile buffers of 37.9 KB: two when the grid has at most one workgroup per
-// compute unit; otherwise one, with a barrier before each restage, so several
-// workgroups share a unit and one's softmax and staging overlap the others'
-// matrix work.  The value MFMA's k index is the lane's own 8 probabilities:
-// slot 8 kq + j is position 16 (j / 4) + 4 kq + j % 4 of the tile, the order
-// V^T is staged in.
+// bf16 products (kBf: every launch at head_dim 128; head_dim 64 keeps the
+// fp32 instruction above): K, V, q and p are each the exact sum of three
+// bf16 pieces (x with its low 16 bits cleared, the same of the rest, the
+// rest: at most 8 significant bits each), staged once per tile by the
+// thread that loaded them.  Two tile buffers (111 KB) when the grid has at
+// most one workgroup per compute unit (16-token decode blocks of the 8B
+// shape); otherwise one (56.8 KB, a barrier before each restage), so two
+// workgroups share a unit and one's softmax and staging overlap the other's
+// matrix work: 8B prefill of 4096 tokens 1339 -> 1107 us, 64 decode tokens
+// 100 -> 79 us.  v_mfma_f32_16x16x32_bf16 takes 32 dims (scores)
+// or the tile's 32 positions (values) per instruction in half the cycles of
+// the fp32 instruction's 4.  Scores and values each keep the 6 piece
+// products above 2^-21 relative: with pieces below 2^-7 and 2^-14 of the
+// value, the dropped three are below 2^-20 |a b| (16 u) a product; for
+// scores within the gamma_{hd+1} score bound with the fp32 sums, for values
+// 16 u of sum_j p_j |v_jd| on top of the fp32 sums' (n + 6) u (the
+// (n + 22) u the tests hold the tiles to).  The value MFMA's k index is the
+// lane's own 8 probabilities: slot 8 kq + j is position 16 (j / 4) + 4 kq +
+// j % 4 of the tile, the order V^T is staged in.
 #include "mlk_attention.h"
 
 #include <cmath>
@@ -110,130 +106,76 @@ struct KvTile {
     }
 };
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-constexpr int kPad = 8;             // fp16 padding per K plane row (rows 16 bytes apart in bank terms)
-constexpr int kVLd = kPfTile + 8;   // V^T plane row: 32 slots + 8 padding
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+constexpr int kBfKLd = 8;  // bf16 padding per K plane row (rows 16 bytes apart in bank terms)
+constexpr int kBfVLd = kPfTile + 8;  // V^T plane row: 32 slots + 8 padding
 
 // K planes [piece][32 positions][HD + 8] and V^T planes [piece][HD][40] of
-// a tile, fp16, and the waves' largest K and V magnitudes of the next tile.
+// a tile, bf16: NBUF buffers (one: 56.8 KB, two workgroups per compute unit).
 template <int HD, int NBUF>
-struct __align__(16) PrefillSmemF16 {
-    uint16_t k[NBUF][2 * kPfTile * (HD + kPad)];
-    uint16_t v[NBUF][2 * HD * kVLd];
-    uint32_t most[2][4];
+struct __align__(16) PrefillSmemBf {
+    uint16_t k[NBUF][3 * kPfTile * (HD + kBfKLd)];
+    uint16_t v[NBUF][3 * HD * kBfVLd];
 };
 
-// 4 floats times s as two fp16 pieces, 4 per dword pair (low half first).
-__device__ inline void Split4(f32x4 x, float s, uint2 (&o)[2]) {
-    h2 hi[2], lo[2];
+// The three bf16 pieces of 4 floats, 4 per dword pair (low half first).
+__device__ inline void SplitPieces4(f32x4 x, uint2 (&o)[3]) {
+    uint32_t h[4], m[4], l[4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const float a = x[2 * i], b = x[2 * i + 1];
-        hi[i].x = static_cast<_Float16>(a * s);
-        hi[i].y = static_cast<_Float16>(b * s);
-        lo[i].x = static_cast<_Float16>(fmaf(a, s, -static_cast<float>(hi[i].x)));
-        lo[i].y = static_cast<_Float16>(fmaf(b, s, -static_cast<float>(hi[i].y)));
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t u = __float_as_uint(x[i]);
+        const float r = x[i] - __uint_as_float(u & 0xFFFF0000u);
+        const uint32_t ru = __float_as_uint(r);
+        h[i] = u;
+        m[i] = ru;
+        l[i] = __float_as_uint(r - __uint_as_float(ru & 0xFFFF0000u));
     }
-    o[0] = make_uint2(__builtin_bit_cast(uint32_t, hi[0]), __builtin_bit_cast(uint32_t, hi[1]));
-    o[1] = make_uint2(__builtin_bit_cast(uint32_t, lo[0]), __builtin_bit_cast(uint32_t, lo[1]));
+    o[0] = make_uint2(__builtin_amdgcn_perm(h[1], h[0], 0x07060302u),
+                      __builtin_amdgcn_perm(h[3], h[2], 0x07060302u));
+    o[1] = make_uint2(__builtin_amdgcn_perm(m[1], m[0], 0x07060302u),
+                      __builtin_amdgcn_perm(m[3], m[2], 0x07060302u));
+    o[2] = make_uint2(__builtin_amdgcn_perm(l[1], l[0], 0x07060302u),
+                      __builtin_amdgcn_perm(l[3], l[2], 0x07060302u));
 }
 
-// 8 floats times s as the pieces' operands.
-__device__ inline void Split8(f32x4 a, f32x4 b, float s, h8 (&o)[2]) {
-    uint2 pa[2], pb[2];
-    Split4(a, s, pa);
-    Split4(b, s, pb);
+// The three pieces of 8 floats as bf16x8 operands.
+__device__ inline void SplitPieces8(f32x4 a, f32x4 b, bf16x8 (&o)[3]) {
+    uint2 pa[3], pb[3];
+    SplitPieces4(a, pa);
+    SplitPieces4(b, pb);
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-        o[p] = __builtin_bit_cast(h8, make_uint4(pa[p].x, pa[p].y, pb[p].x, pb[p].y));
+    for (int p = 0; p < 3; ++p) {
+        const uint4 w = make_uint4(pa[p].x, pa[p].y, pb[p].x, pb[p].y);
+        o[p] = __builtin_bit_cast(bf16x8, w);
     }
 }
 
-// Magnitudes as unsigned keys: twice the bits plus 2^24, which wraps for
-// infinities and NaNs to below every finite value's key, so the largest key
-// is the largest finite magnitude's.
-__device__ inline uint32_t MagKey(float x) { return (__float_as_uint(x) << 1) + 0x01000000u; }
-
-template <int N>
-__device__ inline uint32_t MagKeys(const f32x4 (&x)[N]) {
-    uint32_t m = 0;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = max(m, MagKey(x[i][e]));
-    }
-    return m;
-}
-
-// Largest over the wave, in every lane (uniform).
-__device__ inline uint32_t WaveMaxU32(uint32_t v) {
-#define MLK_DPP_MAX(ctrl, rows)                                                              \
-    v = max(v, static_cast<uint32_t>(__builtin_amdgcn_update_dpp(                            \
-                   static_cast<int>(v), static_cast<int>(v), ctrl, rows, 0xF, false)))
-    MLK_DPP_MAX(0xB1, 0xF);   // quad_perm 1 0 3 2
-    MLK_DPP_MAX(0x4E, 0xF);   // quad_perm 2 3 0 1
-    MLK_DPP_MAX(0x141, 0xF);  // row_half_mirror
-    MLK_DPP_MAX(0x140, 0xF);  // row_mirror
-    MLK_DPP_MAX(0x142, 0xA);  // row_bcast15 into rows 1, 3
-    MLK_DPP_MAX(0x143, 0xC);  // row_bcast31 into rows 2, 3
-#undef MLK_DPP_MAX
-    return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
-}
-
-// The power of two that brings the key's magnitude into [2^14, 2^15) (at
-// most 2^126), and its inverse.
-struct MagScale {
-    int fe;  // the inverse's exponent field, 1 .. 240
-    float s, f;
-    __device__ explicit MagScale(uint32_t key) {
-        const int e = static_cast<int>(key >> 24) - 1;  // the exponent field, -1 .. 254
-        const int b = 268 - e < 253 ? 268 - e : 253;
-        fe = 254 - b;
-        s = __uint_as_float(static_cast<uint32_t>(b) << 23);
-        f = __uint_as_float(static_cast<uint32_t>(fe) << 23);
-    }
-};
-
-// 2^(e - 127), 0 below the smallest normal.
-__device__ inline float Pow2Field(int e) {
-    return __uint_as_float(static_cast<uint32_t>(e > 0 ? e : 0) << 23);
-}
-
-// The next tile for the fp16 kernel: thread tid holds one 4 x 4 block of K
+// The next tile for the bf16 kernel: thread tid holds one 4 x 4 block of K
 // and one of V, at positions 4 a .. 4 a + 3 and dims 4 c4 .. 4 c4 + 3
-// (head_dim 128).  K takes a = tid / 32, c4 = tid % 32 (a 16-lane group
-// writes 128 contiguous bytes of a plane row); V takes a = tid % 8, c4 =
-// tid / 8, so a group's V^T writes (8 position groups x 2 dim rows, 80 bytes
-// apart) meet each LDS bank once.  Positions past load_pos read its row.
-struct KvBlock {
+// (head_dim 128), positions past max_pos reading max_pos's row.  K takes
+// a = tid / 32, c4 = tid % 32 (a 16-lane group writes 128 contiguous bytes
+// of a plane row); V takes a = tid % 8, c4 = tid / 8, so a group's V^T
+// writes (8 position groups x 2 dim rows, 80 bytes apart) meet each LDS
+// bank once.
+struct KvBlockBf {
     f32x4 k[4], v[4];
     const float* kb;
     const float* vb;
-    int64_t slot, load_pos;
+    int64_t slot, max_pos;
     __device__ void Load(int64_t p0) {
         const int tid = static_cast<int>(threadIdx.x);
         const int ak = tid / 32, ck = tid % 32, av = tid % 8, cv = tid / 8;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int64_t p = p0 + 4 * ak + r;
-            const int64_t pos = p <= load_pos ? p : load_pos;
+            const int64_t pos = p <= max_pos ? p : max_pos;
             k[r] = *reinterpret_cast<const f32x4*>(kb + pos * slot + 4 * ck);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int64_t p = p0 + 4 * av + r;
-            const int64_t pos = p <= load_pos ? p : load_pos;
+            const int64_t pos = p <= max_pos ? p : max_pos;
             v[r] = *reinterpret_cast<const f32x4*>(vb + pos * slot + 4 * cv);
-        }
-    }
-    // V at positions past mp (within the tile) is zero: their probabilities
-    // are 0, whatever a later token's V holds
-    __device__ void DropV(int64_t mp) {
-        const int av = static_cast<int>(threadIdx.x) % 8;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            if (4 * av + r > mp) v[r] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
     // K rows 4 a + r; V^T rows 4 c4 + e at slots s0 .. s0 + 3, where
@@ -241,129 +183,108 @@ struct KvBlock {
     // 4 kq + j % 4)
     // KL / VLD: the K and V^T plane row strides (the LDS layout's, or the
     // unpadded images of KvPieces)
-    template <int KL = 128 + kPad, int VLD = kVLd>
-    __device__ void Store(uint16_t* ks, uint16_t* vs, float k_scale, float v_scale) const {
+    template <int KL = 128 + kBfKLd, int VLD = kBfVLd>
+    __device__ void Store(uint16_t* ks, uint16_t* vs) const {
         constexpr int HD = 128;
         const int tid = static_cast<int>(threadIdx.x);
         const int a = tid / 32, c4 = tid % 32, av = tid % 8, cv = tid / 8;
         const int s0 = av < 4 ? 8 * av : 8 * (av - 4) + 4;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            uint2 pc[2];
-            Split4(k[r], k_scale, pc);
+            uint2 pc[3];
+            SplitPieces4(k[r], pc);
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
+            for (int p = 0; p < 3; ++p) {
                 *reinterpret_cast<uint2*>(ks + (p * kPfTile + 4 * a + r) * KL + 4 * c4) = pc[p];
             }
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            uint2 pc[2];
-            Split4(f32x4{v[0][e], v[1][e], v[2][e], v[3][e]}, v_scale, pc);
+            uint2 pc[3];
+            SplitPieces4(f32x4{v[0][e], v[1][e], v[2][e], v[3][e]}, pc);
 #pragma unroll
-            for (int p = 0; p < 2; ++p) {
+            for (int p = 0; p < 3; ++p) {
                 *reinterpret_cast<uint2*>(vs + (p * HD + 4 * cv + e) * VLD + s0) = pc[p];
             }
         }
     }
 };
 
-// The tile's largest K and V keys: each wave's into most[][wave], and after a
-// barrier the largest of the four.
-__device__ inline void PutMost(uint32_t (&most)[2][4], const KvBlock& t) {
-    const uint32_t k = WaveMaxU32(MagKeys(t.k)), v = WaveMaxU32(MagKeys(t.v));
-    if (threadIdx.x % kWave == 0) {
-        most[0][threadIdx.x / kWave] = k;
-        most[1][threadIdx.x / kWave] = v;
-    }
-}
-__device__ inline uint32_t GetMost(const uint32_t (&most)[4]) {
-    const uint4 m = *reinterpret_cast<const uint4*>(most);
-    return __builtin_amdgcn_readfirstlane(max(max(m.x, m.y), max(m.z, m.w)));
-}
-
 // Pre-split tiles (head_dim 128): per KV head g and tile t of 32 cache
-// positions, the K planes [2][32][128] and the V^T planes [2][128][32] in
-// fp16, exactly what KvBlock::Store writes to LDS, without the row padding:
-// one 32 KB image a tile, images of head g at g * n_tiles + t, then the
-// tiles' largest K and V keys (uint2 each, in the same order).  A prompt
-// chunk's workgroups each stage every tile of their prefix, so the split
-// (most of the VALU work of a tile) is done once here instead of once per 16
-// tokens.
-constexpr int kPieceHalves = 2 * kPfTile * 128;          // fp16 of a K (or V^T) image
+// positions, the K planes [3][32][128] and the V^T planes [3][128][32] in
+// bf16, exactly what KvBlockBf::Store writes to LDS, without the row
+// padding: one 48 KB image a tile, images of head g at g * n_tiles + t.
+// A prompt chunk's workgroups each stage every tile of their prefix, so
+// the split (most of the VALU work of a tile) is done once here instead of
+// once per 16 tokens.
+constexpr int kPieceHalves = 3 * kPfTile * 128;        // bf16 of a K (or V^T) image
 constexpr int kPieceTileU4 = 2 * kPieceHalves * 2 / 16;  // uint4 of a tile's two images
 
 __global__ __launch_bounds__(kPfThreads) void KvPieces(const float* __restrict__ kc,
                                                        const float* __restrict__ vc,
                                                        int64_t slot, int KV, int64_t max_pos,
                                                        int64_t n_tiles,
-                                                       uint16_t* __restrict__ images,
-                                                       uint2* __restrict__ keys) {
-    __shared__ __align__(16) uint32_t most[2][4];
+                                                       uint16_t* __restrict__ images) {
     const int64_t t = blockIdx.x / KV;
     const int g = static_cast<int>(blockIdx.x % KV);
-    KvBlock tile;
+    KvBlockBf tile;
     tile.kb = kc + static_cast<int64_t>(g) * 128;
     tile.vb = vc + static_cast<int64_t>(g) * 128;
     tile.slot = slot;
-    tile.load_pos = max_pos;  // positions past it read its row
+    tile.max_pos = max_pos;  // positions past it read its row
     tile.Load(t * kPfTile);
-    PutMost(most, tile);
-    __syncthreads();
-    const uint32_t kk = GetMost(most[0]), kv = GetMost(most[1]);
-    const int64_t at = static_cast<int64_t>(g) * n_tiles + t;
-    uint16_t* ks = images + at * (2 * kPieceHalves);
-    tile.Store<128, kPfTile>(ks, ks + kPieceHalves, MagScale(kk).s, MagScale(kv).s);
-    if (threadIdx.x == 0) keys[at] = make_uint2(kk, kv);
+    uint16_t* ks = images + (static_cast<int64_t>(g) * n_tiles + t) * (2 * kPieceHalves);
+    tile.Store<128, kPfTile>(ks, ks + kPieceHalves);
 }
 
 // The next tile from KvPieces' images: thread tid copies uint4 tid + 256 i
-// (i < 4) of the K image and of the V^T image.  K image uint4 u: piece
+// (i < 6) of the K image and of the V^T image.  K image uint4 u: piece
 // u / 512, row (u / 16) % 32, dims 8 (u % 16) ..; V^T image: piece u / 512,
-// dim (u / 4) % 128, slots 8 (u % 4) ...
+// dim (u / 4) % 128, slots 8 (u % 4) ...  In the workgroup's last tile, V
+// at positions past its last token's is zeroed (their probabilities are 0;
+// KvBlockBf reads the last token's row there, so finite values give the
+// same sums), and K there needs nothing (those scores are replaced by -inf).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 struct KvBlockPre {
-    u32x4 k[4], v[4];   // native vectors, not uint4 structs (see KvTile::Load)
-    uint2 key;
+    u32x4 k[6], v[6];   // native vectors, not uint4 structs (see KvTile::Load)
     const u32x4* base;  // head g's first image
-    const uint2* keys;  // and its key
+    int64_t max_pos;
     __device__ void Load(int64_t p0) {
         const u32x4* src = base + (p0 / kPfTile) * kPieceTileU4;
         const int tid = static_cast<int>(threadIdx.x);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 6; ++i) {
             k[i] = src[tid + kPfThreads * i];
             v[i] = src[kPieceTileU4 / 2 + tid + kPfThreads * i];
         }
-        key = keys[p0 / kPfTile];
-    }
-    // as KvBlock::DropV
-    __device__ void DropV(int64_t mp) {
+        const int64_t mp = max_pos - p0;  // the last position kept, within the tile
+        if (mp < kPfTile - 1) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            // slots 8 q4 + 2d, + 1 (dword d): positions 16 (d / 2) + 4 q4 +
-            // 2 (d % 2), + 1
-            const int64_t b = 4 * ((threadIdx.x + kPfThreads * i) % 4);
-            const auto keep = [&](int64_t pl) {
-                return (pl <= mp ? 0x0000FFFFu : 0u) | (pl + 1 <= mp ? 0xFFFF0000u : 0u);
-            };
-            v[i].x &= keep(b);
-            v[i].y &= keep(b + 2);
-            v[i].z &= keep(b + 16);
-            v[i].w &= keep(b + 18);
+            for (int i = 0; i < 6; ++i) {
+                // slots 8 q4 + 2d, + 1 (dword d): positions 16 (d / 2) + 4 q4 +
+                // 2 (d % 2), + 1
+                const int64_t b = 4 * ((tid + kPfThreads * i) % 4);
+                const auto keep = [&](int64_t pl) {
+                    return (pl <= mp ? 0x0000FFFFu : 0u) | (pl + 1 <= mp ? 0xFFFF0000u : 0u);
+                };
+                v[i].x &= keep(b);
+                v[i].y &= keep(b + 2);
+                v[i].z &= keep(b + 16);
+                v[i].w &= keep(b + 18);
+            }
         }
     }
-    __device__ void Store(uint16_t* ks, uint16_t* vs, float, float) const {
-        constexpr int KL = 128 + kPad;
+    __device__ void Store(uint16_t* ks, uint16_t* vs) const {
+        constexpr int KL = 128 + kBfKLd;
         const int tid = static_cast<int>(threadIdx.x);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 6; ++i) {
             const int u = tid + kPfThreads * i;
             *reinterpret_cast<u32x4*>(ks + ((u / 512) * kPfTile + (u / 16) % kPfTile) * KL +
                                       8 * (u % 16)) = k[i];
-            *reinterpret_cast<u32x4*>(vs + ((u / 512) * 128 + (u / 4) % 128) * kVLd + 8 * (u % 4)) =
-                v[i];
+            *reinterpret_cast<u32x4*>(vs + ((u / 512) * 128 + (u / 4) % 128) * kBfVLd +
+                                      8 * (u % 4)) = v[i];
         }
     }
 };
@@ -380,21 +301,20 @@ struct TileChunks {
     int32_t* err;
 };
 
-template <int HD, bool kChunked, bool kF16, int NBUF = 2, bool kPre = false>
+template <int HD, bool kChunked, bool kBf, int NBUF = 2, bool kPre = false>
 __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
     const float* __restrict__ q, int64_t q_stride, const float* __restrict__ kc,
     const float* __restrict__ vc, int64_t slot, int KV, int H, int32_t pos0, int64_t T,
     float scale, float* __restrict__ out, int head_blocks, TileChunks tc,
-    const uint16_t* __restrict__ images, const uint2* __restrict__ image_keys,
-    int64_t n_image_tiles, uint32_t* __restrict__ a_planes) {
+    const uint16_t* __restrict__ images, int64_t n_image_tiles, uint32_t* __restrict__ a_planes) {
 #pragma clang fp contract(off)
-    static_assert(!kF16 || HD == 128, "fp16 products: head_dim 128");
-    static_assert(!kPre || kF16, "pre-split tiles: fp16 products");
-    static_assert(NBUF == 2 || (NBUF == 1 && kF16), "one tile buffer: fp16 products only");
+    static_assert(!kBf || HD == 128, "bf16 products: head_dim 128");
+    static_assert(!kPre || kBf, "pre-split tiles: bf16 products");
+    static_assert(NBUF == 2 || (NBUF == 1 && kBf), "one tile buffer: bf16 products only");
     constexpr int LD = HD + 4;
     constexpr int NC = HD / 16;                          // 16-dim chunks
-    constexpr int KL = HD + kPad;                        // K plane row (fp16)
-    __shared__ typename std::conditional<kF16, PrefillSmemF16<HD, NBUF>, PrefillSmem<HD>>::type sm;
+    constexpr int KL = HD + kBfKLd;                      // K plane row (bf16)
+    __shared__ typename std::conditional<kBf, PrefillSmemBf<HD, NBUF>, PrefillSmem<HD>>::type sm;
     const int group = H / KV;
     const int64_t n_tb = (T + kPfTokens - 1) / kPfTokens;
     int64_t bid = blockIdx.x;
@@ -445,28 +365,17 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
         }
     }
 
-    f32x4 qv[NC];        // fp32: dims 16 c + 4 kq .. + 3
-    h8 qp[2][HD / 32];   // fp16: pieces of dims 32 c + 8 kq .. + 7
-    float q_factor = 1.0f;
-    if constexpr (kF16) {
+    f32x4 qv[NC];         // fp32: dims 16 c + 4 kq .. + 3
+    bf16x8 qp[3][HD / 32];  // bf16: pieces of dims 32 c + 8 kq .. + 7
+    if constexpr (kBf) {
         const float* qrow = q + t * q_stride + static_cast<int64_t>(h) * HD + 8 * kq;
-        f32x4 qr[2 * (HD / 32)];
 #pragma unroll
         for (int c = 0; c < HD / 32; ++c) {
-            qr[2 * c] = *reinterpret_cast<const f32x4*>(qrow + 32 * c);
-            qr[2 * c + 1] = *reinterpret_cast<const f32x4*>(qrow + 32 * c + 4);
-        }
-        uint32_t key = MagKeys(qr);  // the row's, over its 4 lanes
-        key = max(key, static_cast<uint32_t>(__shfl_xor(static_cast<int>(key), 16, kWave)));
-        key = max(key, static_cast<uint32_t>(__shfl_xor(static_cast<int>(key), 32, kWave)));
-        const MagScale ms(key);
-        q_factor = ms.f;
+            bf16x8 pc[3];
+            SplitPieces8(*reinterpret_cast<const f32x4*>(qrow + 32 * c),
+                         *reinterpret_cast<const f32x4*>(qrow + 32 * c + 4), pc);
 #pragma unroll
-        for (int c = 0; c < HD / 32; ++c) {
-            h8 pc[2];
-            Split8(qr[2 * c], qr[2 * c + 1], ms.s, pc);
-            qp[0][c] = pc[0];
-            qp[1][c] = pc[1];
+            for (int p = 0; p < 3; ++p) qp[p][c] = pc[p];
         }
     } else {
         const float* qrow = q + t * q_stride + static_cast<int64_t>(h) * HD + 4 * kq;
@@ -475,49 +384,19 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
     }
 
     typename std::conditional<kPre, KvBlockPre,
-                              typename std::conditional<kF16, KvBlock, KvTile<HD>>::type>::type
+                              typename std::conditional<kBf, KvBlockBf, KvTile<HD>>::type>::type
         tile;
     if constexpr (kPre) {
         tile.base = reinterpret_cast<const u32x4*>(images) +
                     static_cast<int64_t>(g) * n_image_tiles * kPieceTileU4;
-        tile.keys = image_keys + static_cast<int64_t>(g) * n_image_tiles;
     } else {
         tile.kb = kc + static_cast<int64_t>(g) * HD;
         tile.vb = vc + static_cast<int64_t>(g) * HD;
         tile.slot = slot;
-        if constexpr (kF16) {
-            // a prompt chunk's tiles as KvPieces reads them, to the chunk's
-            // last token, so their scales are the images'
-            tile.load_pos = kChunked ? max_pos : pos0 + T - 1;
-        } else {
-            tile.max_pos = max_pos;
-        }
     }
+    tile.max_pos = max_pos;
     auto load = [&](int64_t p0) { tile.Load(p0); };
-    // fp16: true K = stored K * k_factor, true V = stored V * 2^(v_exp - 127)
-    float k_factor = 1.0f;
-    int v_exp = 127;
-    // the tile at p0 from its registers into buffer buf (fp16 without images:
-    // after PutMost and a barrier)
-    auto store = [&](int buf, int64_t p0) {
-        if constexpr (kF16) {
-            uint32_t kk, kv;
-            if constexpr (kPre) {
-                kk = __builtin_amdgcn_readfirstlane(tile.key.x);
-                kv = __builtin_amdgcn_readfirstlane(tile.key.y);
-            } else {
-                kk = GetMost(sm.most[0]);
-                kv = GetMost(sm.most[1]);
-            }
-            const MagScale mk(kk), mv(kv);
-            k_factor = mk.f;
-            v_exp = mv.fe;
-            if ((kPre || !kChunked) && max_pos - p0 < kPfTile - 1) tile.DropV(max_pos - p0);
-            tile.Store(sm.k[buf], sm.v[buf], mk.s, mv.s);
-        } else {
-            tile.Store(sm.k[buf], sm.v[buf]);
-        }
-    };
+    auto store = [&](int buf) { tile.Store(sm.k[buf], sm.v[buf]); };
 
     f32x4 acc[NC];  // O^T: acc[c][r] = dim 16c + 4 kq + r of query i16
 #pragma unroll
@@ -527,16 +406,11 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
 
     const int64_t n_tiles = (p_end - p_begin + kPfTile - 1) / kPfTile;
     load(p_begin);
-    if constexpr (kF16 && !kPre) {
-        PutMost(sm.most, tile);
-        __syncthreads();
-    }
-    store(0, p_begin);
+    store(0);
     __syncthreads();
-    int unit = v_exp;  // fp16: true sums = acc * 2^(unit - 127) * 2^-14
     // positions fit in 32 bits (below max_seq); log2-unit score scale
     const int32_t my_pos_32 = static_cast<int32_t>(my_pos);
-    const float scale2 = scale * 1.44269504088896340736f * q_factor;
+    const float scale2 = scale * 1.44269504088896340736f;
     for (int64_t it = 0; it < n_tiles; ++it) {
         const int buf = NBUF == 2 ? static_cast<int>(it & 1) : 0;
         const int32_t p0_32 = static_cast<int32_t>(p_begin + it * kPfTile);
@@ -550,15 +424,22 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
 #pragma unroll
             for (int pt = 0; pt < 2; ++pt) {
                 s[pt] = f32x4{0.f, 0.f, 0.f, 0.f};
-                if constexpr (kF16) {
+                if constexpr (kBf) {
                     const uint16_t* krow = &sm.k[buf][(pt * 16 + i16) * KL + 8 * kq];
 #pragma unroll
                     for (int c = 0; c < HD / 32; ++c) {
-                        const h8 k0 = *reinterpret_cast<const h8*>(krow + 32 * c);
-                        const h8 k1 = *reinterpret_cast<const h8*>(krow + kPfTile * KL + 32 * c);
-                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k1, qp[0][c], s[pt], 0, 0, 0);
-                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qp[1][c], s[pt], 0, 0, 0);
-                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k0, qp[0][c], s[pt], 0, 0, 0);
+                        bf16x8 kp[3];
+#pragma unroll
+                        for (int p = 0; p < 3; ++p) {
+                            kp[p] = *reinterpret_cast<const bf16x8*>(krow + p * kPfTile * KL + 32 * c);
+                        }
+                        // the 6 largest piece products, smallest first
+                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[2], qp[0][c], s[pt], 0, 0, 0);
+                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], qp[2][c], s[pt], 0, 0, 0);
+                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], qp[1][c], s[pt], 0, 0, 0);
+                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[1], qp[0][c], s[pt], 0, 0, 0);
+                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], qp[1][c], s[pt], 0, 0, 0);
+                        s[pt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kp[0], qp[0][c], s[pt], 0, 0, 0);
                     }
                 } else {
                     const float* krow = &sm.k[buf][(pt * 16 + i16) * LD + 4 * kq];
@@ -581,9 +462,7 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
                 for (int r = 0; r < 4; ++r) {
                     // scores in log2 units (scale * log2(e)), for exp2 below
                     const int32_t pos = p0_32 + pt * 16 + 4 * kq + r;
-                    // (fp16: K's factor, then q's with the scale)
-                    const float sr = kF16 ? s[pt][r] * k_factor : s[pt][r];
-                    const float x = pos <= my_pos_32 ? sr * scale2 : -INFINITY;
+                    const float x = pos <= my_pos_32 ? s[pt][r] * scale2 : -INFINITY;
                     sv[pt * 4 + r] = x;
                     tmax = fmaxf(tmax, x);
                 }
@@ -597,19 +476,12 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
             const float mnew = fmaxf(m, tmax);
             const float mref = kChunked && mnew == -INFINITY ? 0.0f : mnew;
             // rescale only when some query's max moved (the factor is then
-            // exactly 1 for the others: skipping it changes nothing), or the
-            // accumulators' unit grows to this V tile's
+            // exactly 1 for the others: skipping it changes nothing)
             if (__builtin_amdgcn_ballot_w64(mnew != m) != 0) {
                 const float corr = __builtin_amdgcn_exp2f(m - mref);
                 l *= corr;
 #pragma unroll
                 for (int c = 0; c < NC; ++c) acc[c] *= corr;
-            }
-            if (kF16 && v_exp > unit) {
-                const float grow = Pow2Field(127 + unit - v_exp);
-#pragma unroll
-                for (int c = 0; c < NC; ++c) acc[c] *= grow;
-                unit = v_exp;
             }
             float pv[8];
 #pragma unroll
@@ -618,19 +490,25 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
                 l += pv[i];
             }
             m = mnew;
-            if constexpr (kF16) {
+            if constexpr (kBf) {
                 // B: this lane's probabilities, slot j = position 16 (j / 4) + 4 kq + j % 4
-                h8 pp[2];
-                Split8(f32x4{pv[0], pv[1], pv[2], pv[3]}, f32x4{pv[4], pv[5], pv[6], pv[7]},
-                       Pow2Field(127 + 14 + v_exp - unit), pp);
+                bf16x8 pp[3];
+                SplitPieces8(f32x4{pv[0], pv[1], pv[2], pv[3]}, f32x4{pv[4], pv[5], pv[6], pv[7]}, pp);
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
-                    const uint16_t* vrow = &sm.v[buf][(16 * c + i16) * kVLd + 8 * kq];
-                    const h8 v0 = *reinterpret_cast<const h8*>(vrow);
-                    const h8 v1 = *reinterpret_cast<const h8*>(vrow + HD * kVLd);
-                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v1, pp[0], acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v0, pp[1], acc[c], 0, 0, 0);
-                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v0, pp[0], acc[c], 0, 0, 0);
+                    const uint16_t* vrow = &sm.v[buf][(16 * c + i16) * kBfVLd + 8 * kq];
+                    bf16x8 vp[3];
+#pragma unroll
+                    for (int p = 0; p < 3; ++p) {
+                        vp[p] = *reinterpret_cast<const bf16x8*>(vrow + p * HD * kBfVLd);
+                    }
+                    // the 6 piece products above 2^-21 relative, smallest first
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[2], pp[0], acc[c], 0, 0, 0);
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[2], acc[c], 0, 0, 0);
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[1], acc[c], 0, 0, 0);
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[1], pp[0], acc[c], 0, 0, 0);
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[1], acc[c], 0, 0, 0);
+                    acc[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vp[0], pp[0], acc[c], 0, 0, 0);
                 }
             } else {
 #pragma unroll
@@ -647,17 +525,13 @@ __global__ __launch_bounds__(kPfThreads) void AttnPrefill(
                 }
             }
         }
-        const int64_t p_next = p_begin + (it + 1 < n_tiles ? it + 1 : it) * kPfTile;
-        if constexpr (kF16 && !kPre) PutMost(sm.most, tile);
-        // one buffer: every wave is done with the tile before it is replaced;
-        // fp16 without images: the next tile's largest magnitudes are known
-        if constexpr (NBUF == 1 || (kF16 && !kPre)) __syncthreads();
-        store(NBUF == 1 ? 0 : buf ^ 1, p_next);
+        if constexpr (NBUF == 1) {
+            __syncthreads();  // every wave is done with the tile before it is replaced
+            store(0);
+        } else {
+            store(buf ^ 1);
+        }
         __syncthreads();
-    }
-    if constexpr (kF16) {  // out of the fp16 unit
-#pragma unroll
-        for (int c = 0; c < NC; ++c) acc[c] = acc[c] * (1.0f / 16384.0f) * Pow2Field(unit);
     }
     l += __shfl_xor(l, 16, kWave);
     l += __shfl_xor(l, 32, kWave);
@@ -711,24 +585,21 @@ bool PrefillSupported(int32_t head_dim, const float* q, int64_t q_row_stride, co
 
 int64_t PrefillImageBytes(int32_t n_kv_heads, int32_t head_dim, int64_t n_pos) {
     if (head_dim != 128 || n_kv_heads <= 0 || n_pos <= 0) return 0;
-    // a tile's image and its two keys (rounded up to 16 bytes)
-    return static_cast<int64_t>(n_kv_heads) * ((n_pos + kPfTile - 1) / kPfTile) *
-           (kPieceTileU4 * 16 + 16);
+    return static_cast<int64_t>(n_kv_heads) * ((n_pos + kPfTile - 1) / kPfTile) * kPieceTileU4 *
+           16;
 }
 
 namespace {
 
-// K and V of positions 0 .. n_pos - 1 into tile images and keys at `images`
-// (PrefillImageBytes).
+// K and V of positions 0 .. n_pos - 1 into tile images (PrefillImageBytes).
 mlk_status LaunchPieces(const float* kc, const float* vc, int64_t slot, int32_t KV, int64_t n_pos,
-                        uint16_t* images, uint2** keys, int64_t* n_tiles, hipStream_t s) {
+                        uint16_t* images, int64_t* n_tiles, hipStream_t s) {
     *n_tiles = (n_pos + kPfTile - 1) / kPfTile;
     if (*n_tiles * KV > 0x7FFFFFFF) {
         return Fail(MLK_ERR_INVALID, "attention prefill: launch too large");
     }
-    *keys = reinterpret_cast<uint2*>(images + *n_tiles * KV * (2 * kPieceHalves));
     hipLaunchKernelGGL(KvPieces, dim3(static_cast<unsigned>(*n_tiles * KV)), dim3(kPfThreads), 0, s,
-                       kc, vc, slot, KV, n_pos - 1, *n_tiles, images, *keys);
+                       kc, vc, slot, KV, n_pos - 1, *n_tiles, images);
     return CheckLaunch("KvPieces");
 }
 
@@ -750,27 +621,25 @@ mlk_status LaunchPrefill(const float* q, int64_t q_row_stride, const float* kc, 
     // (positions 0 .. pos0 + T - 1), then stage the images
     const int64_t n_pos = pos0 + T;
     const int64_t image_bytes = PrefillImageBytes(KV, head_dim, n_pos);
-    if (image_bytes > 0 && T >= kPrefillImageMinTokens && workspace != nullptr &&
-        Aligned(workspace, 16) &&
-        static_cast<int64_t>(workspace_bytes) >= image_bytes) {
+    if (image_bytes > 0 && PrefillImages(T, pos0) && workspace != nullptr &&
+        Aligned(workspace, 16) && static_cast<int64_t>(workspace_bytes) >= image_bytes) {
         uint16_t* images = static_cast<uint16_t*>(workspace);
-        uint2* keys = nullptr;
         int64_t n_tiles = 0;
-        const mlk_status st = LaunchPieces(kc, vc, slot, KV, n_pos, images, &keys, &n_tiles, s);
+        const mlk_status st = LaunchPieces(kc, vc, slot, KV, n_pos, images, &n_tiles, s);
         if (st != MLK_OK) return st;
         hipLaunchKernelGGL((AttnPrefill<128, false, true, 1, true>), grid, dim3(kPfThreads), 0, s,
                            q, q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
-                           none, images, keys, n_tiles, a_planes);
+                           none, images, n_tiles, a_planes);
         return CheckLaunch("AttnPrefill");
     }
     if (head_dim == 64) {
         hipLaunchKernelGGL((AttnPrefill<64, false, false>), grid, dim3(kPfThreads), 0, s, q,
                            q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
-                           none, nullptr, nullptr, 0, a_planes);
+                           none, nullptr, 0, a_planes);
     } else {
         hipLaunchKernelGGL((AttnPrefill<128, false, true, 1>), grid, dim3(kPfThreads), 0, s, q,
                            q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
-                           none, nullptr, nullptr, 0, a_planes);
+                           none, nullptr, 0, a_planes);
     }
     return CheckLaunch("AttnPrefill");
 }
@@ -818,27 +687,26 @@ mlk_status LaunchDecodeTile(const float* q, int64_t q_row_stride, const float* k
     if (head_dim == 64) {
         hipLaunchKernelGGL((AttnPrefill<64, true, false>), grid, dim3(kPfThreads), 0, s, q,
                            q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
-                           tc, nullptr, nullptr, 0, nullptr);
+                           tc, nullptr, 0, nullptr);
     } else if (images_at != nullptr) {
         // (consecutive positions) tiles from images, as LaunchPrefill
         uint16_t* images = static_cast<uint16_t*>(images_at);
-        uint2* keys = nullptr;
         int64_t n_tiles = 0;
-        const mlk_status st =
-            LaunchPieces(kc, vc, slot, KV, pos0 + T, images, &keys, &n_tiles, s);
+        const mlk_status st = LaunchPieces(kc, vc, slot, KV, pos0 + T, images, &n_tiles, s);
         if (st != MLK_OK) return st;
         hipLaunchKernelGGL((AttnPrefill<128, true, true, 1, true>), grid, dim3(kPfThreads), 0, s, q,
                            q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
-                           tc, images, keys, n_tiles, nullptr);
+                           tc, images, n_tiles, nullptr);
     } else if (blocks <= ComputeUnits()) {
-        // two tile buffers (76 KB of LDS)
+        // bf16 products: their 111 KB of LDS leave one workgroup per unit,
+        // which a grid this small uses anyway
         hipLaunchKernelGGL((AttnPrefill<128, true, true>), grid, dim3(kPfThreads), 0, s, q,
                            q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
-                           tc, nullptr, nullptr, 0, nullptr);
+                           tc, nullptr, 0, nullptr);
     } else {
         hipLaunchKernelGGL((AttnPrefill<128, true, true, 1>), grid, dim3(kPfThreads), 0, s, q,
                            q_row_stride, kc, vc, slot, KV, H, pos0, T, scale, out, head_blocks,
-                           tc, nullptr, nullptr, 0, nullptr);
+                           tc, nullptr, 0, nullptr);
     }
     return CheckLaunch("AttnPrefill (decode tokens)");
 }

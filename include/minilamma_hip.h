@@ -259,16 +259,15 @@ int64_t mlk_attention_workspace_bytes(int64_t n_tokens, int32_t n_heads, int32_t
  * bytes (chunk partials); out must not alias q.  Sums are fp32 in the
  * kernel's order (the reference's tolerance: 2e-5 against float64,
  * test/cuda_attention_test.cc:108-109); with head_dim 128, batches of 5 or
- * more tokens and the prefill kernel form each q.k and p.v product from three
- * products of fp16 pieces: K, V, q and p to within 2^-23 of each value (and
- * 2^-39 of the largest of the 32 positions' K or V, or of the q row), so a
- * product is within 2^-20 of its exact value (fp32 rounds at 2^-24).  With
- * positions == NULL, 16 or more tokens, head_dim 64 or 128 and 16-byte aligned
- * q rows, out and caches, the call runs mlk_attention_prefill_f32's kernel;
- * from 128 tokens at head_dim 128, a 16-byte aligned workspace of at least
- * 12 * KV * head_dim * (pos0 + n_tokens rounded up to 32) bytes lets it split
- * K and V into fp16 pieces once (one extra launch) instead of in every
- * workgroup, with the same results.  From max_ctx 2048, when the chunk's
+ * more tokens and the prefill kernel form each q.k and p.v product from the
+ * six bf16 piece products above 2^-21 relative, so each product is within
+ * 2^-20 of its exact value (fp32 rounds at 2^-24).  With positions == NULL, 16
+ * or more tokens, head_dim 64 or 128 and 16-byte aligned q rows, out and
+ * caches, the call runs mlk_attention_prefill_f32's kernel; at head_dim 128,
+ * from 1024 tokens and from 384 after at least as many positions, a 16-byte
+ * aligned workspace of at least 12 * KV * head_dim * (pos0 + n_tokens rounded
+ * up to 32) bytes lets it split K and V into bf16 pieces once (one extra
+ * launch) instead of in every workgroup, with the same results.  From max_ctx 2048, when the chunk's
  * blocks of 16 tokens are too few to fill the device, a 16-byte aligned
  * workspace of mlk_attention_workspace_bytes() lets it split the positions
  * over workgroups, partial sums merged as for decode tokens (the images then
@@ -367,9 +366,9 @@ typedef struct {
 /* Device bytes of the workspace of mlk_forward_layer_batch for n_tokens
  * tokens attending up to max_ctx positions; consecutive_positions != 0 when
  * the call passes positions == NULL (0 on bad input).  A prompt chunk of
- * 128 or more tokens at head_dim 128 includes the attention's pre-split
- * K/V (up to 12 bytes per cached K and V element of a layer up to max_ctx);
- * one of few tokens over 2048 or more positions, the attention's partial
+ * 1024 or more tokens, or 384 after as many positions, at head_dim 128 includes
+ * the attention's pre-split K/V (12 bytes per cached element pair of a layer up
+ * to max_ctx, rounded up to 32 positions); one of few tokens over 2048 or more positions, the attention's partial
  * sums. */
 int64_t mlk_forward_layer_workspace_bytes(const mlk_layer_config* cfg, int64_t n_tokens,
                                           int64_t max_ctx, int32_t consecutive_positions);

@@ -611,13 +611,9 @@ def test_attention_tiles_dropped_pieces_within_bound(mlk):
 
 @pytest.mark.parametrize("T,pos0", [(16, 64), (33, 63), (128, 37), (200, 0)])
 def test_attention_tiles_of_far_apart_magnitudes(mlk, T, pos0):
-    """The fp16 pieces' scales: 32-position tiles whose K and V differ by up to
-    2^126, one of them zero, and a zero query row; through the prefill kernel
-    (T below and from the images' 128 tokens, ragged last blocks) and the
-    shared decode tiles.  Each V and p is within 2^-39 of its tile's largest
-    (of 1), on top of its own 2^-23: at most 2^-38 (n + 1) M more than the
-    tiles' bound, M the KV head's largest |V| up to the end of the tile of the
-    token block's last position."""
+    """32-position tiles whose K and V differ by up to 2^126, one of them zero,
+    and a zero query row; through the prefill kernel (ragged last blocks) and
+    the shared decode tiles, to the tiles' own bound."""
     rng = np.random.default_rng(T + pos0)
     H, KV, hd = 8, 2, 128
     S = pos0 + T
@@ -631,12 +627,8 @@ def test_attention_tiles_of_far_apart_magnitudes(mlk, T, pos0):
     q[T // 2] = 0.0
     ex, pav, dmax, n = prefill_exact(q, kc, vc, 1, pos0)
 
-    def more(last, tokens):
-        m = np.abs(vc[1, :last // 32 * 32 + 32]).max(axis=(0, 2)).astype(np.float64)
-        return 2.0 ** -38 * (tokens + 1) * np.repeat(m, H // KV)[:, None]
-
-    def check(got, t, last, what):
-        bound = (2 * dmax[t][:, None] + (n[t] + 22) * U) * pav[t] + more(last, n[t]) + 1e-30
+    def check(got, t, what):
+        bound = (2 * dmax[t][:, None] + (n[t] + 22) * U) * pav[t] + 1e-30
         assert np.isfinite(got).all(), f"{what}: non-finite output"
         err = np.abs(got.astype(np.float64) - ex[t])
         assert (err <= bound).all(), f"{what} token {t}: worst {float((err / bound).max()):.3g}"
@@ -644,18 +636,77 @@ def test_attention_tiles_of_far_apart_magnitudes(mlk, T, pos0):
     for images in (False, True):
         got = run_prefill(mlk, cache, q, 1, pos0, images=images)
         for t in range(T):
-            check(got[t], t, min(pos0 + t // 16 * 16 + 15, S - 1), f"images {images}")
+            check(got[t], t, f"images {images}")
     pos = np.sort(rng.choice(np.arange(pos0, S), 16, replace=False)).astype(np.int32)
     got = cache.attend(q[pos - pos0], 1, pos)
     for i, p in enumerate(pos):
-        check(got[i], p - pos0, S - 1, "decode tiles")
+        check(got[i], p - pos0, "decode tiles")
+
+
+@pytest.mark.parametrize("H,KV,T,pos0", [(8, 2, 40, 70), (4, 1, 400, 410), (4, 2, 64, 2100)])
+def test_attention_large_values_leave_others_alone(mlk, H, KV, T, pos0):
+    """Finite K and V far above the rest: in dims that other dims share a tile
+    with, at an early position (its probability is 0 or not), and at later
+    positions, which a token does not attend.  The other dims and the earlier
+    tokens keep the tiles' bound, whole and split over positions, from images
+    or not, and through the shared decode tiles.  Large finite K whose scores
+    are small through small q stay finite."""
+    rng = np.random.default_rng(T + pos0)
+    hd, S = 128, pos0 + T
+    kc, vc = random_cache(rng, 1, S, KV, hd)
+    vc[0, 3, :, 64:] = 1e12
+    vc[0, 40, :, 32:64] = -1e20
+    kc[0, 5] = 0
+    kc[0, 5, :, 0] = -300  # (q's first dim is 8 below)
+    vc[0, 5] = 1e30
+    cut = T // 2 + 3
+    kc[0, pos0 + cut:, :, 7] = 1e8
+    vc[0, pos0 + cut:] *= 1e12
+    q = rng.standard_normal((T, H, hd)).astype(np.float32)
+    q[..., 0] = 8
+    cache = Cache(mlk, kc, vc)
+    ex, pav, dmax, n = prefill_exact(q, kc, vc, 0, pos0)
+    dm = np.empty((cut, H))  # the scores' bound without position 5
+    k5 = kc.copy()
+    k5[0, 5] = 0
+    dm[:] = prefill_exact(q[:cut], k5, vc, 0, pos0)[2]
+    n_pos = pos0 + T
+    part = (mlk.attention_workspace_bytes(T, H, KV, hd, n_pos) + 255) // 256 * 256
+    d_q = mlk.DeviceBuffer.from_array(q)
+    got = {"whole": run_prefill(mlk, cache, q, 0, pos0)}
+    for name, size in (("partials", part), ("images", part + image_bytes(KV, n_pos))):
+        out = mlk.DeviceBuffer.empty((T, H, hd))
+        ws = mlk.DeviceBuffer(max(size, 4) + 256, np.uint8)
+        ws.upload(np.full(ws.nbytes, 0xA5, np.uint8))
+        mlk.attention_decode(d_q, cache.k, cache.v, 1, S, H, KV, hd, 0, T, out, n_pos, pos0=pos0,
+                             workspace=ws, workspace_bytes=size)
+        got[name] = out.download()
+        np.testing.assert_array_equal(ws.download()[size:], np.full(ws.nbytes - size, 0xA5))
+    for i in range(0, cut - 15, 16):  # 16 decode tokens share a tile
+        pos = np.arange(pos0 + i, pos0 + i + 16, dtype=np.int32)
+        got.setdefault("decode", np.zeros((T, H, hd), np.float32))[i:i + 16] = cache.attend(
+            q[i:i + 16], 0, pos)
+    for name, o in got.items():
+        m = cut // 16 * 16 if name == "decode" else cut
+        bound = (2 * dm[:m, :, None] + (n[:m, None, None] + 22) * U) * pav[:m] + 1e-30
+        err = np.abs(o[:m].astype(np.float64) - ex[:m])
+        assert (err <= bound).all(), f"{name}: {float((err / bound).max()):.3g} times the bound"
+    kc[0, pos0 + cut:] = 0
+    kc *= np.float32(2.0 ** 104)
+    q *= np.float32(2.0 ** -112)
+    vc[:] = rng.standard_normal(vc.shape)
+    ex, pav, dmax, n = prefill_exact(q, kc, vc, 0, pos0)
+    assert_prefill_close(run_prefill(mlk, Cache(mlk, kc, vc), q, 0, pos0), ex, pav, dmax, n,
+                         "large K, small q", pieces=True)
 
 
 @pytest.mark.parametrize("H,KV,hd,T,pos0,spare", [
     (8, 2, 128, 16, 2032, 0),     # 2048 positions: the first split context
     (8, 2, 128, 17, 2030, 0),     # 2047: whole, the prefill entry's sums
-    (12, 2, 128, 127, 2500, 0),   # the last size without images; a partly idle head block
-    (8, 2, 128, 128, 2483, 9000), # images behind the partials; max_ctx far past the chunk
+    (12, 2, 128, 127, 2500, 0),   # a partly idle head block
+    (8, 2, 128, 128, 2483, 9000), # max_ctx far past the chunk
+    (4, 1, 128, 383, 2483, 0),    # the last size without images behind the partials
+    (4, 1, 128, 384, 2483, 9000), # and the first with them
     (8, 8, 64, 33, 2300, 40),     # head_dim 64, ragged blocks
 ])
 def test_attention_prefill_split_over_positions(mlk, H, KV, hd, T, pos0, spare):
