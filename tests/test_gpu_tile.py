@@ -36,6 +36,8 @@ def run(mlk, orc, kind, x, w, bias=None, workspace="auto"):
     T, K = x.shape
     out = w.shape[0]
     B = mlk.DeviceBuffer.from_array
+    if workspace == "auto" and T < 8:  # (the wrapper's "auto" takes none)
+        workspace = mlk.DeviceBuffer(max(mlk.linear_workspace_bytes(T, K, out), 16), np.uint8)
     y = mlk.DeviceBuffer.empty((T, out))
     b = None if bias is None else B(bias)
     if kind == "f32":
@@ -291,3 +293,41 @@ def test_few_row_layer_matches_oracle(orc, mlk, wt, T, gaps):
     x = dm.hidden(tokens, positions=pos if gaps else None)
     got = dm.logits(x, T).download().astype(np.float64)
     assert (np.abs(got - want) <= 1e-5 + 1e-4 * np.abs(want)).all()
+
+
+@pytest.mark.parametrize("T", [4, 7])
+def test_few_rows_need_no_shared_workspace(mlk, orc, T):
+    """Calls below 8 rows with the wrapper's default workspace share no buffer
+    and allocate nothing: the first one can be captured, and calls on two
+    streams at once give the sums of calls one after another."""
+    out, K = 14336, 4096
+    assert mlk.linear_workspace_bytes(T, K, out) > 0  # (one would be used)
+    rng = np.random.default_rng(T)
+    blocks = rng.integers(0, 256, (out, K // 32, 34), dtype=np.uint8)
+    blocks[..., 1] = 0x20  # scales about 2^-7
+    d_w = mlk.DeviceBuffer.from_array(blocks)
+    xs = [mlk.DeviceBuffer.from_array(normal(rng, (T, K))) for _ in range(2)]
+    ys = [mlk.DeviceBuffer.empty((T, out)) for _ in range(2)]
+    streams = [mlk.Stream(), mlk.Stream()]
+
+    def call(i):
+        mlk.linear_quant("q8_0", xs[i], d_w, ys[i], T, K, out, stream=streams[i])
+
+    with mlk.Graph.capture(streams[0]) as graph:
+        call(0)
+    want = []
+    for i in range(2):
+        call(i)
+        streams[i].synchronize()
+        want.append(ys[i].download())
+    for _ in range(20):
+        call(0)
+        call(1)
+    for _ in range(3):
+        graph.launch()
+        call(1)
+    for s in streams:
+        s.synchronize()
+    for i in range(2):
+        np.testing.assert_array_equal(ys[i].download(), want[i])
+    graph.close()
