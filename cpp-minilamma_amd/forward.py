@@ -187,6 +187,8 @@ class DeviceModel:
         d_pos = None
         if positions is not None:
             positions = np.ascontiguousarray(positions, np.int32)
+            if positions.size < T:
+                raise ValueError(f"{positions.size} positions for {T} tokens")
             d_pos = DeviceBuffer.from_array(positions)
             max_ctx = int(positions.max()) + 1
         else:
@@ -245,8 +247,10 @@ class DeviceModel:
         if positions is None:
             d_pos, max_ctx = None, pos0 + T
         else:
-            positions = np.ascontiguousarray(positions, np.int32)
-            ids_pos[at[1] // 4:at[1] // 4 + T] = positions.ravel()[:T]
+            positions = np.ascontiguousarray(positions, np.int32).ravel()
+            if positions.size < T:
+                raise ValueError(f"{positions.size} positions for {T} tokens")
+            ids_pos[at[1] // 4:at[1] // 4 + T] = positions[:T]
             max_ctx = int(positions.max()) + 1
         check(lib.mlk_memcpy(buf.ptr, ids_pos.ctypes.data, ids_pos.nbytes, H2D), "upload")
         self._embed(ids, T, x, stream)

@@ -87,6 +87,18 @@ def test_forward_scratch_is_kept_across_calls(mlk, fwd):
     assert dm._scratch is None
 
 
+def test_forward_refuses_too_few_positions(fwd):
+    """One position is not taken for every token; extra ones are left alone."""
+    model, tokens, positions, logits = tiny_model()
+    dm = fwd.DeviceModel(model)
+    for n in (1, len(tokens) - 1):
+        for call in (dm.forward, dm.hidden):
+            with pytest.raises(ValueError, match="positions"):
+                call(tokens, positions=np.arange(n, dtype=np.int32))
+    longer = np.arange(len(tokens) + 3, dtype=np.int32)
+    np.testing.assert_array_equal(dm.forward(tokens, positions=longer), dm.forward(tokens))
+
+
 CASES = [  # config overrides, weight type, biases, tokens in the prefill batch
     (dict(dim=256, hidden_dim=512, n_heads=4, n_kv_heads=2, head_dim=64), "f32", True, 40),
     (dict(dim=256, hidden_dim=512, n_heads=4, n_kv_heads=2, head_dim=64), "q8_0", True, 40),
