@@ -922,7 +922,7 @@ mlk_status AttentionDecode(const float* q, int64_t q_row_stride, const float* k_
     if (prompt && !prompt_split) {
         // a prompt chunk at consecutive positions: the matrix-core prefill
         // kernel (a workspace of PrefillImageBytes holds the pre-split tiles)
-        // (and a's planes, when asked, for a tiled wo)
+        // (and a's planes, when asked, for a planar wo)
         if (planes != nullptr && planes_written != nullptr) *planes_written = true;
         return LaunchPrefill(q, q_row_stride, k_cache + layer * max_seq * slot,
                              v_cache + layer * max_seq * slot, slot, n_heads, n_kv_heads,

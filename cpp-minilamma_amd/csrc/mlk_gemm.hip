@@ -465,8 +465,6 @@ constexpr int kSkRows = 64;  // output rows per workgroup (16 per wave)
 // A lane's weights of one K chunk, and the chunk offset of the inputs its
 // k-slot takes in stage u (8 consecutive inputs per stage; A and B use the
 // same assignment, so each product x[t, k] * w[o, k] is formed once).
-//   F32    4 stages of 32 inputs: the lane's k-slot q reads 8q .. 8q + 7 of
-//          each 32 (two 16-byte non-temporal loads per stage).
 //   Q8_0 / Q4_0 / Q4_1   8 stages: the lane owns a piece, the two blocks 2q
 //          and 2q + 1 of the 8-block chunk (68 / 36 / 40 bytes, 4-byte
 //          aligned, read as 16-byte loads), and stage u takes its inputs
@@ -475,24 +473,6 @@ typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
 
 template <int WT>
 struct WChunk;
-
-template <>
-struct WChunk<kWF32> {
-    static constexpr int kStages = 4;
-    static constexpr bool kPieces = false;
-    f32x4 a[kStages], b[kStages];
-    __device__ void Load(const uint8_t* w, int64_t row, int64_t row_bytes, int64_t k0, int q) {
-#pragma unroll
-        for (int u = 0; u < kStages; ++u) {
-            const f32x4* p =
-                reinterpret_cast<const f32x4*>(w + row * row_bytes) + (k0 + 32 * u + 8 * q) / 4;
-            a[u] = __builtin_nontemporal_load(p);
-            b[u] = __builtin_nontemporal_load(p + 1);
-        }
-    }
-    __device__ float Get(int u, int j) const { return j < 4 ? a[u][j & 3] : b[u][j & 3]; }
-    __device__ static int XOff(int u, int q) { return 32 * u + 8 * q; }
-};
 
 template <int QT>
 struct PieceChunk {
@@ -1210,18 +1190,18 @@ __global__ __launch_bounds__(kGemmThreads) void SplitKReduceFused(const float* _
     }
 }
 
-int SkinnyChunk(int wt) { return wt == kWF32 ? 32 * WChunk<kWF32>::kStages : 32 * 8; }
+constexpr int64_t kSkChunk = 32 * 8;  // inputs of a chunk
 
 // Chunks per workgroup: two for quantized weights when K is a multiple of
 // two chunks, else one.
 int SkinnyPieces(int wt, int64_t T, int64_t K) {
-    return wt != kWF32 && T <= 32 && K % (2 * SkinnyChunk(wt)) == 0 ? 2 : 1;
+    return wt != kWF32 && T <= 32 && K % (2 * kSkChunk) == 0 ? 2 : 1;
 }
 
 // The skinny kernel takes SkinnyPieces chunks per workgroup: K / (that many
 // chunks) splits.
 SplitPlan PlanSkinny(int wt, int64_t T, int64_t K) {
-    const int64_t chunk = SkinnyChunk(wt) * SkinnyPieces(wt, T, K);
+    const int64_t chunk = kSkChunk * SkinnyPieces(wt, T, K);
     SplitPlan p;
     p.per_split = chunk;
     p.splits = static_cast<int>(K / chunk);
@@ -1232,7 +1212,7 @@ SplitPlan PlanSkinny(int wt, int64_t T, int64_t K) {
 // layer's projections: the quantized types up to 32 rows (F32 stays tiled).
 bool SkinnyApplies(int wt, int64_t T, int64_t K) {
     const bool rows = wt >= MLK_Q8_0 && wt <= MLK_Q4_1 && T <= 32;
-    return rows && K % SkinnyChunk(wt) == 0 && K / SkinnyChunk(wt) <= 4096;
+    return rows && K % kSkChunk == 0 && K / kSkChunk <= 4096;
 }
 
 template <int TT, int NP>
@@ -1251,11 +1231,7 @@ void LaunchSkinnyT(int wt, dim3 grid, hipStream_t s, const float* x, const Skinn
             hipLaunchKernelGGL((GemmSkinny<MLK_Q4_1, TT, NP>), grid, dim3(kSkThreads), 0, s, x, a,
                                T, K, row_bytes, partial);
             break;
-        default:
-            if constexpr (NP == 1) {
-                hipLaunchKernelGGL((GemmSkinny<kWF32, TT, 1>), grid, dim3(kSkThreads), 0, s, x, a,
-                                   T, K, row_bytes, partial);
-            }
+        default:  // (SkinnyApplies names no other)
             break;
     }
 }
@@ -1298,13 +1274,19 @@ void LaunchTiles(int wt, dim3 grid, hipStream_t s, const float* x, const uint8_t
             hipLaunchKernelGGL((GemmMfma<MLK_Q4_1, BM>), grid, dim3(kGemmThreads), 0, s, x, w,
                                bias, y, T, K, O, row_bytes, tiles_m, tiles, per_split, partial);
             break;
-        case kWPlanarQ8:
-            hipLaunchKernelGGL((GemmMfma<kWPlanarQ8, BM>), grid, dim3(kGemmThreads), 0, s, x, w,
-                               bias, y, T, K, O, row_bytes, tiles_m, tiles, per_split, partial);
+        case kWPlanarQ8:  // more than 32 rows of more than 2^22 inputs (LinearPlanar, TileApplies)
+            if constexpr (BM > 32) {
+                hipLaunchKernelGGL((GemmMfma<kWPlanarQ8, BM>), grid, dim3(kGemmThreads), 0, s, x,
+                                   w, bias, y, T, K, O, row_bytes, tiles_m, tiles, per_split,
+                                   partial);
+            }
             break;
-        case kWPlanarQ4:
-            hipLaunchKernelGGL((GemmMfma<kWPlanarQ4, BM>), grid, dim3(kGemmThreads), 0, s, x, w,
-                               bias, y, T, K, O, row_bytes, tiles_m, tiles, per_split, partial);
+        case kWPlanarQ4:  // more than 32 rows of more than 2^22 inputs (LinearPlanar, TileApplies)
+            if constexpr (BM > 32) {
+                hipLaunchKernelGGL((GemmMfma<kWPlanarQ4, BM>), grid, dim3(kGemmThreads), 0, s, x,
+                                   w, bias, y, T, K, O, row_bytes, tiles_m, tiles, per_split,
+                                   partial);
+            }
             break;
         default:
             hipLaunchKernelGGL((GemmMfma<kWF32, BM>), grid, dim3(kGemmThreads), 0, s, x, w, bias,
