@@ -331,3 +331,71 @@ def test_few_rows_need_no_shared_workspace(mlk, orc, T):
     for i in range(2):
         np.testing.assert_array_equal(ys[i].download(), want[i])
     graph.close()
+
+
+@pytest.mark.parametrize("wt", ["q8_0", "f32"])
+def test_tile_layer_epilogues_of_marked_rows(mlk, orc, wt):
+    """Rows with a value far above the rest through a layer whose gate/up and wo
+    launches are not split over K, so SwiGLU and the residual add run in the
+    tiles, some of them with more marked rows than are summed one by one:
+    every row to 4e-6 of its float64 value (2-norm; four times what 256- to
+    3072-term fp32 sums show here)."""
+    import importlib
+    fwd = importlib.import_module(mlk.__name__ + ".forward")
+    D, F, H, KV, hd, T = 256, 3072, 2, 1, 128, 1024
+    rng = np.random.default_rng(9)
+    shapes = dict(wq=(H * hd, D), wk=(KV * hd, D), wv=(KV * hd, D), wo=(D, H * hd),
+                  w_gate=(F, D), w_up=(F, D), w_down=(D, F))
+    lw, kept, w64 = fwd.LayerWeights(), [], {}
+    g = [1 + normal(rng, (D,), 0.1) for _ in range(2)]
+    d_g = [mlk.DeviceBuffer.from_array(v) for v in g]
+    lw.attention_norm, lw.ffn_norm = (b.ptr for b in d_g)
+    for n, (o, i) in shapes.items():
+        w = normal(rng, (o, i), 0.06)
+        lin = fwd.LinearWeight()
+        if wt == "f32":
+            kept.append(mlk.DeviceBuffer.from_array(w))
+            lin.type, w64[n] = fwd.WEIGHT_F32, w.astype(np.float64)
+        else:
+            b = orc.quantize(wt, w)
+            kept.append(mlk.DeviceBuffer.from_array(np.ascontiguousarray(b, np.uint8)))
+            lin.type, w64[n] = mlk.QUANT[wt], orc.dequantize(wt, b, o, i).astype(np.float64)
+        lin.data = kept[-1].ptr
+        setattr(lw, n, lin)
+    x = normal(rng, (T, D))
+    x[::100, 5] = 1e9  # a few rows of a tile
+    x[256:400:3, 9] = 1e7  # many
+    cfg = dict(dim=D, hidden_dim=F, n_heads=H, n_kv_heads=KV, head_dim=hd, rope_type=0,
+               theta=10000.0, eps=1e-5)
+    ws = mlk.DeviceBuffer(fwd.layer_workspace_bytes(cfg, T, T, True), np.uint8)
+    d_x = mlk.DeviceBuffer.from_array(x)
+    kc, vc = (mlk.DeviceBuffer.empty((1, T, KV, hd)) for _ in range(2))
+    fwd.forward_layer_batch(cfg, lw, d_x, T, kc, vc, 1, T, 0, T, ws, pos0=0)
+
+    def norm(a, gain):
+        return a / np.sqrt((a * a).mean(1, keepdims=True) + 1e-5) * gain
+
+    def rope(a):
+        ang = np.arange(T)[:, None] * 10000.0 ** (-2 * np.arange(hd // 2) / hd)
+        c, s = np.cos(ang)[:, None], np.sin(ang)[:, None]
+        e, o = a[..., 0::2], a[..., 1::2]
+        return np.stack([e * c - o * s, e * s + o * c], -1).reshape(a.shape)
+    x64 = x.astype(np.float64)
+    h = norm(x64, g[0])
+    q = rope((h @ w64["wq"].T).reshape(T, H, hd))
+    k = rope((h @ w64["wk"].T).reshape(T, KV, hd))[:, 0]
+    v = h @ w64["wv"].T
+    att = np.empty((T, H, hd))
+    for i in range(H):
+        s = q[:, i] @ k.T / np.sqrt(hd)
+        s[np.triu_indices(T, 1)] = -np.inf
+        p = np.exp(s - s.max(1, keepdims=True))
+        att[:, i] = p / p.sum(1, keepdims=True) @ v
+    y = x64 + att.reshape(T, -1) @ w64["wo"].T
+    h = norm(y, g[1])
+    gate = h @ w64["w_gate"].T
+    y = y + (gate / (1 + np.exp(-gate)) * (h @ w64["w_up"].T)) @ w64["w_down"].T
+    cols = np.setdiff1d(np.arange(D), [5, 9])  # (there the residual's own size hides the sums)
+    err = np.linalg.norm(d_x.download()[:, cols] - y[:, cols], axis=1)
+    rel = err / np.linalg.norm(y[:, cols], axis=1)
+    assert rel.max() < 4e-6, f"row {rel.argmax()}: {rel.max():.3g}"
