@@ -172,11 +172,13 @@ mlk_status mlk_linear_f32(const float* x, const float* w, const float* bias, flo
 /* Device bytes of the optional workspace of mlk_linear_quant / mlk_linear_f32
  * for this shape on the current device (0: the call uses none).  Calls of
  * 8 rows or more, and of 3 or more over large matrices, run on the matrix
- * cores in output tiles; when those tiles are too few to fill the compute units, a workspace of this size
- * (16-byte aligned, not aliasing x, W or y) lets the call split K over
- * workgroups and add the partial sums in a fixed order.  Without it (NULL or
- * smaller) the call is still correct, only slower.  No counterpart in the
- * reference (cuBLAS keeps its own workspace). */
+ * cores in output tiles; when those tiles are too few to fill the compute
+ * units, a workspace of this size (16-byte aligned, not aliasing x, W or y)
+ * lets the call split K over workgroups and add the partial sums in a fixed
+ * order.  Without it (NULL or smaller) the call is still correct, only slower;
+ * 3 to 7 rows of Q4_1 are then summed as d sum(code x) + m sum(x), with the
+ * error of those two sums.  No counterpart in the reference (cuBLAS keeps its
+ * own workspace). */
 int64_t mlk_linear_workspace_bytes(int64_t rows, int64_t in_features, int64_t out_features);
 
 /* Planar layout of Q8_0 / Q4_0 weights [out, in] (in % 256 == 0), made once
